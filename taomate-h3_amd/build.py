@@ -21,7 +21,9 @@ LIB = PKG / "libtaomate_h3_amd.so"
 # Measurement kernels of bench.py's `ceilings` object, kept out of the product library.
 CEILINGS_SRC = "ceilings.hip"
 CEILINGS_LIB = PKG / "libh3q_ceilings.so"
-SOURCES = ["act_quant.hip", "head_quant.hip", "norm_quant.hip", "swiglu_quant.hip", "gemm.hip", "gemm_w4.hip", "gemm_skinny.hip", "capi.hip"]
+SOURCES = ["act_quant.hip", "head_quant.hip", "norm_quant.hip", "swiglu_quant.hip", "gemm.hip", "gemm_w4.hip", "gemm_skinny.hip",
+           "gemm_stream.hip", "gemm_stream_e4m3_tiled.hip", "gemm_stream_e4m3_rows.hip", "gemm_stream_int8_tiled.hip",
+           "gemm_stream_int8_rows.hip", "capi.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

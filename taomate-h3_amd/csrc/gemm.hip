@@ -729,6 +729,9 @@ hipError_t launch_gemm(int kind, bool raw_i32, const GemmArgs& args, hipStream_t
     GemmArgs a = args;
     a.out_vec = (a.ldo % 4 == 0) && (a.n % 4 == 0) && ((uintptr_t)a.out % 16 == 0);
     const bool lora = a.lora_t != nullptr;
+    if (kind != kOpBF16 && !raw_i32) {
+        if (const int tile = stream_tile(a)) return launch_gemm_stream(kind, tile, a, st);
+    }
     if (kind != kOpBF16 && !raw_i32 && skinny_supported(a)) return launch_gemm_skinny(kind, a, st);
     if (kind != kOpBF16 && !raw_i32 && w4_supported(a)) return launch_gemm_w4(kind, a, st);
     if (kind == kOpE4M3)

@@ -114,6 +114,13 @@ constexpr int64_t kSkinnyMaxM = 128;
 bool skinny_supported(const GemmArgs& a);
 hipError_t launch_gemm_skinny(int kind, const GemmArgs& a, hipStream_t st);
 
+// Weight-streaming GEMM over tiles sized to fill the chip (gemm_stream.hpp):
+// scaled e4m3 / int8, any layout, optional bias and rank <= 128 LoRA, n and ldo
+// multiples of 8, a 16-byte aligned output.  stream_tile gives the tile to use
+// (0: another kernel is the better one); launch_gemm routes there itself.
+int stream_tile(const GemmArgs& a);
+hipError_t launch_gemm_stream(int kind, int tile, const GemmArgs& a, hipStream_t st);
+
 // Fused RMSNorm + AdaLN modulate (+ residual gate) + per-token quantization
 // (norm_quant.hip).  All bf16 tensors are row-major with element strides;
 // tables are [T, table_stride] and row r uses table row indices[r].

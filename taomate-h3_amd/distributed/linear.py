@@ -31,6 +31,8 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .. import ops
+from ..inference import fused_kernels, w8a8
+from ..inference.fused_kernels import QuantizedActivations, as_dense
 
 
 def _cross_rank(what: str) -> NotImplementedError:
@@ -43,8 +45,6 @@ def _fp8_w8a8_linear(inputs: torch.Tensor, weight: torch.Tensor, weight_scale: t
                      bias: torch.Tensor | None) -> torch.Tensor:
     """Per-token dynamic e4m3fn activations x per-channel e4m3fn weights
     (the activations may come pre-quantized from a fused producer)."""
-    from ..inference.fused_kernels import QuantizedActivations
-
     shape = (*inputs.shape[:-1], int(weight.shape[0]))
     if isinstance(inputs, QuantizedActivations):
         if inputs.fmt != ops.FMT_E4M3FN:
@@ -53,9 +53,9 @@ def _fp8_w8a8_linear(inputs: torch.Tensor, weight: torch.Tensor, weight_scale: t
                             b_tiled=ops.is_tiled(weight), m=int(inputs.codes.shape[0]))
         return out.reshape(shape)
     flat = inputs.reshape(-1, int(inputs.shape[-1])).contiguous()
-    q, s, a_tiled = ops.quant_activations_for(flat, ops.FMT_E4M3FN, ops.ROUND_DIV, weight)
-    out = ops.scaled_mm(q, weight, s.reshape(-1), weight_scale.reshape(-1), bias=bias, a_tiled=a_tiled,
-                        b_tiled=ops.is_tiled(weight), m=int(flat.shape[0]))
+    tiled = ops.is_tiled(weight)
+    q, s, a_tiled = ops.quant_activations_for(flat, ops.FMT_E4M3FN, ops.ROUND_DIV, weight, tiled=tiled)
+    out = ops.scaled_mm(q, weight, s, weight_scale, bias=bias, a_tiled=a_tiled, b_tiled=tiled, m=int(flat.shape[0]))
     return out.reshape(shape)
 
 
@@ -63,14 +63,12 @@ def _fp8_tensor_linear(inputs: torch.Tensor, weight: torch.Tensor, weight_scale:
                        bias: torch.Tensor | None, input_scale: torch.Tensor | None) -> torch.Tensor:
     """Per-tensor FP8 (FL/distributed/linear.py:80-101): dynamic or static
     activation scale, then the scaled GEMM in place of torch._scaled_mm."""
-    from ..inference.fused_kernels import quantize_fp8_e4m3, quantize_fp8_e4m3_dynamic
-
     shape = (*inputs.shape[:-1], int(weight.shape[0]))
     flat = inputs.reshape(-1, int(inputs.shape[-1]))
     if input_scale is None:
-        q, input_scale = quantize_fp8_e4m3_dynamic(flat)
+        q, input_scale = fused_kernels.quantize_fp8_e4m3_dynamic(flat)
     else:
-        q = quantize_fp8_e4m3(flat, input_scale)
+        q = fused_kernels.quantize_fp8_e4m3(flat, input_scale)
     if bias is not None and bias.dtype != torch.bfloat16:
         bias = bias.to(torch.bfloat16)
     out = ops.scaled_mm(q, weight, input_scale.reshape(1).to(torch.float32),
@@ -82,18 +80,11 @@ def _module_linear(module: nn.Module, inputs: torch.Tensor, bias: torch.Tensor |
     """H3/distributed/linear.py:15-33 plus the FP8 formats.  ``inputs`` may
     also be per-token codes from a fused producer (QuantizedActivations): the
     per-token W8A8 paths consume them directly, the others use their bf16 rows."""
-    from ..inference.fused_kernels import QuantizedActivations, as_dense
-
     if getattr(module, ops.TILED_WEIGHT_ATTR, False):
         ops.module_weight_tiled(module)  # re-marks the storage of a deep-copied tiled weight
     scale = getattr(module, "_cutlass_w8a8_weight_scale", None)
-    if isinstance(inputs, QuantizedActivations) and scale is None and \
-            getattr(module, "_fp8_w8a8_weight_scale", None) is None:
-        inputs = as_dense(inputs)
     if scale is not None:
-        from ..inference.w8a8 import cutlass_w8a8_linear
-
-        return cutlass_w8a8_linear(
+        return w8a8.cutlass_w8a8_linear(
             inputs,
             module.weight,
             scale,
@@ -105,6 +96,7 @@ def _module_linear(module: nn.Module, inputs: torch.Tensor, bias: torch.Tensor |
     fp8_rows = getattr(module, "_fp8_w8a8_weight_scale", None)
     if fp8_rows is not None:
         return _fp8_w8a8_linear(inputs, module.weight, fp8_rows, bias)
+    inputs = as_dense(inputs)
     fp8_tensor = getattr(module, "_fp8_weight_scale", None)
     if fp8_tensor is not None:
         return _fp8_tensor_linear(inputs, module.weight, fp8_tensor, bias, _module_fp8_input_scale(module, inputs))
@@ -120,9 +112,7 @@ def _linear(inputs: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | Non
     if cutlass_w8a8_weight_scale is not None:
         if fp8_weight_scale is not None:
             raise RuntimeError("a linear cannot combine CUTLASS W8A8 with another quantizer")
-        from ..inference.w8a8 import cutlass_w8a8_linear
-
-        return cutlass_w8a8_linear(inputs, weight, cutlass_w8a8_weight_scale, bias=bias,
+        return w8a8.cutlass_w8a8_linear(inputs, weight, cutlass_w8a8_weight_scale, bias=bias,
                                    workspace=cutlass_w8a8_workspace, weight_t=cutlass_w8a8_weight_t,
                                    weight_scale_t=cutlass_w8a8_weight_scale_t)
     if fp8_weight_scale is None:

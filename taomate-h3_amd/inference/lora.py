@@ -27,6 +27,7 @@ import torch
 import torch.nn.functional as F
 
 from .. import ops
+from .fused_kernels import as_dense
 
 FUSED_MAX_RANK = 128
 
@@ -51,33 +52,33 @@ def _fusable(base: Any, lora_a: torch.Tensor, lora_b: torch.Tensor) -> bool:
 def fused_quantized_lora_linear(base: Any, inputs: torch.Tensor, lora_a: torch.Tensor, lora_b: torch.Tensor,
                                 scale: float) -> torch.Tensor:
     """base(x) + scale * (x @ A^T) @ B^T with one bf16 rounding, for a W8A8 base."""
-    shape = (*inputs.shape[:-1], int(base.weight.shape[0]))
-    ops.module_weight_tiled(base)  # re-marks the storage of a deep-copied tiled weight
+    weight = base.weight
+    shape = (*inputs.shape[:-1], int(weight.shape[0]))
+    tiled = ops.module_weight_tiled(base)  # re-marks the storage of a deep-copied tiled weight
     flat = inputs.reshape(-1, int(inputs.shape[-1]))
     if flat.dtype != torch.bfloat16:
         flat = flat.to(torch.bfloat16)
     flat = flat.contiguous()
     t = ops.lora_down(flat, lora_a.contiguous())
     bias = getattr(base, "bias", None)
-    if getattr(base, "_cutlass_w8a8_weight_scale", None) is not None:
+    w_scale = getattr(base, "_cutlass_w8a8_weight_scale", None)
+    if w_scale is not None:
         if bias is not None:
             raise RuntimeError("H3 W8A8 supports bias-free linears only")
         workspace = getattr(base, "_cutlass_w8a8_workspace", None)
         if workspace is not None:
-            _, s, out = workspace.buffers(flat, int(base.weight.shape[0]))
+            _, s, out = workspace.buffers(flat, int(weight.shape[0]))
             q = workspace._codes_buffer(flat)
         else:
             q = s = out = None
-        q, s, a_tiled = ops.quant_activations_for(flat, ops.FMT_INT8, ops.ROUND_RCP_MUL, base.weight, codes=q,
-                                                  scales=s, lora=True)
-        w_scale = base._cutlass_w8a8_weight_scale
+        q, s, a_tiled = ops.quant_activations_for(flat, ops.FMT_INT8, ops.ROUND_RCP_MUL, weight, codes=q, scales=s,
+                                                  lora=True, tiled=tiled)
     else:
-        q, s, a_tiled = ops.quant_activations_for(flat, ops.FMT_E4M3FN, ops.ROUND_DIV, base.weight, lora=True)
+        q, s, a_tiled = ops.quant_activations_for(flat, ops.FMT_E4M3FN, ops.ROUND_DIV, weight, lora=True, tiled=tiled)
         out = None
         w_scale = base._fp8_w8a8_weight_scale
-    out = ops.scaled_mm(q, base.weight, s.reshape(-1), w_scale.reshape(-1), bias=bias, lora_t=t,
-                        lora_b=lora_b.contiguous(), lora_scale=float(scale), out=out, a_tiled=a_tiled,
-                        b_tiled=ops.module_weight_tiled(base), m=int(flat.shape[0]))
+    out = ops.scaled_mm(q, weight, s, w_scale.reshape(-1), bias=bias, lora_t=t, lora_b=lora_b.contiguous(),
+                        lora_scale=float(scale), out=out, a_tiled=a_tiled, b_tiled=tiled, m=int(flat.shape[0]))
     return out.reshape(shape)
 
 
@@ -106,8 +107,6 @@ class H3InferenceParallelLinearLoRA(torch.nn.Module):
         self.register_buffer("lora_b", b, persistent=False)
 
     def forward(self, inputs: torch.Tensor) -> torch.Tensor:
-        from .fused_kernels import as_dense
-
         if not self.adapter_enabled:
             return self.base(inputs)
         if self.kind == "row" and int(getattr(self.base, "tp_size", 1)) > 1:

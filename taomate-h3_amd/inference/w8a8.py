@@ -33,6 +33,7 @@ from typing import Any
 import torch
 
 from .. import _lib, ops
+from .fused_kernels import QuantizedActivations
 
 INTERIOR_FC1_QKV_POLICY = "interior_fc1_qkv_v1"
 _STREAM_LOAD_TEMPORARY_BYTES = 8 * 1024 * 1024
@@ -214,6 +215,9 @@ class CutlassW8A8Workspace:
 
     @staticmethod
     def _stream(inputs: torch.Tensor) -> tuple[int | None, int]:
+        if inputs.is_cuda:
+            index = inputs.get_device()
+            return index, ops._raw_stream(index)
         stream = torch.cuda.current_stream(device=inputs.device)
         return inputs.device.index, int(stream.cuda_stream)
 
@@ -242,12 +246,14 @@ class CutlassW8A8Workspace:
 
     def linear(self, inputs: torch.Tensor, weight_t: torch.Tensor, weight_scale_t: torch.Tensor) -> torch.Tensor:
         rows = int(inputs.shape[0])
-        _, activation_scale, output = self.buffers(inputs, int(weight_t.shape[1]))
+        weight = weight_t.t()
+        tiled = ops.is_tiled(weight)
+        _, activation_scale, output = self.buffers(inputs, int(weight.shape[0]))
         quantized, activation_scale, a_tiled = ops.quant_activations_for(
-            inputs, ops.FMT_INT8, ops.ROUND_RCP_MUL, weight_t, codes=self._codes_buffer(inputs),
-            scales=activation_scale)
-        ops.scaled_mm(quantized, weight_t.t(), activation_scale, weight_scale_t.reshape(-1), out=output,
-                      a_tiled=a_tiled, b_tiled=ops.is_tiled(weight_t), m=rows)
+            inputs, ops.FMT_INT8, ops.ROUND_RCP_MUL, weight, codes=self._codes_buffer(inputs),
+            scales=activation_scale, tiled=tiled)
+        ops.scaled_mm(quantized, weight, activation_scale, weight_scale_t.reshape(-1), out=output, a_tiled=a_tiled,
+                      b_tiled=tiled, m=rows)
         return output
 
 
@@ -258,8 +264,6 @@ def cutlass_w8a8_linear(inputs: torch.Tensor, weight: torch.Tensor, weight_scale
     (H3/inference/w8a8.py:190-220)."""
     if bias is not None:
         raise RuntimeError("H3 W8A8 supports bias-free linears only")
-    from .fused_kernels import QuantizedActivations
-
     if isinstance(inputs, QuantizedActivations):
         return _linear_from_codes(inputs, weight, weight_scale, workspace)
     shape = (*inputs.shape[:-1], int(weight.shape[0]))

@@ -13,7 +13,7 @@ import weakref
 
 import torch
 
-from . import _lib
+from . import _lib, _native
 
 FMT_E4M3FN = 0
 FMT_INT8 = 1
@@ -29,7 +29,25 @@ QUOTIENT_TRITON = 1
 SKINNY_MAX_M = 128   # rows up to which the weight-streaming GEMM runs
 
 _CODE_DTYPES = {FMT_E4M3FN: torch.float8_e4m3fn, FMT_INT8: torch.int8}
+_OUT_F16 = {torch.bfloat16: False, torch.float16: True}
 _FORMATS = {torch.float8_e4m3fn: FMT_E4M3FN, torch.int8: FMT_INT8}
+
+
+# The functions below try the native wrapper first (csrc/torch_ops.cpp: the same
+# checks, allocations and entry point).  It declines anything out of the
+# ordinary, and the Python body then checks the same arguments and raises.
+_raw_stream = torch._C._cuda_getCurrentRawStream
+
+
+def _native_call(name: str, first: torch.Tensor, *args):
+    """The native wrapper's result, or None when it declines (or ``first`` is not on a GPU)."""
+    device = first.get_device()
+    if device < 0:
+        return None
+    try:
+        return getattr(_native.module(), name)(first, *args, _raw_stream(device))
+    except TypeError:  # an argument that is no tensor or number
+        return None
 
 
 def _stream(t: torch.Tensor) -> ctypes.c_void_p:
@@ -68,6 +86,9 @@ def code_dtype(fmt: int) -> torch.dtype:
 def quant_rows(x: torch.Tensor, fmt: int, rounding: int = ROUND_DIV, *, codes: torch.Tensor | None = None,
                scales: torch.Tensor | None = None) -> tuple[torch.Tensor, torch.Tensor]:
     """Per-row quantization of bf16 ``x [rows, K]`` -> (codes [rows, K], scales [rows, 1] fp32)."""
+    got = _native_call("quant_rows", x, fmt, rounding, codes, scales)
+    if got is not None:
+        return got
     _require_gpu("quant_rows", x, codes, scales)
     _rows_2d("quant_rows x", x, torch.bfloat16)
     rows, cols = x.shape
@@ -111,6 +132,12 @@ def norm_modulate_quant(value: torch.Tensor, weight: torch.Tensor, scale: torch.
     allocate one, None/False for none.  ``fmt``: code format for the per-token
     quantization (None: no codes).  Returns (out or None, codes or None,
     scales or None)."""
+    if codes is None and scales is None and not isinstance(out, torch.Tensor):
+        gated = (None, None, None) if residual_gate is None else residual_gate
+        got = _native_call("norm_modulate_quant", value, weight, scale, shift, indices, eps,
+                           -1 if fmt is None else fmt, rounding, out is True, *gated)
+        if got is not None:
+            return got
     branch = gate = hidden = None
     if residual_gate is not None:
         branch, gate, hidden = residual_gate
@@ -200,7 +227,7 @@ def _unmark(key: tuple[str, int, int], ref: weakref.ref) -> None:
 
 def is_tiled(t: torch.Tensor | None) -> bool:
     """True when ``t`` (or any view of the same storage) holds tiled codes."""
-    if t is None or not isinstance(t, torch.Tensor) or t.device.type == "meta":
+    if not _TILED_STORAGES or t is None or not isinstance(t, torch.Tensor) or t.is_meta:
         return False
     ref = _TILED_STORAGES.get(_storage_key(t))
     return ref is not None and ref() is t.untyped_storage()
@@ -258,19 +285,20 @@ def check_layout(name: str, t: torch.Tensor, tiled: bool) -> None:
 
 def quant_activations_for(x: torch.Tensor, fmt: int, rounding: int, weight: torch.Tensor, *,
                           codes: torch.Tensor | None = None, scales: torch.Tensor | None = None,
-                          lora: bool = False):
+                          lora: bool = False, tiled: bool | None = None):
     """Per-token quantization of the 2-D activations of a linear whose weight
     codes are ``weight`` (bf16 output): tiled when the weight is tiled and the
     GEMM reads tiled activations at this shape -- the weight-streaming GEMM
     for at most 128 tokens (no LoRA), the four-wave GEMM above that (K >= 256,
     N a multiple of 8, with or without the LoRA epilogue) -- else row-major.
     Returns (codes, scales, a_tiled); ``codes`` may be a larger workspace
-    buffer of rows >= tiled_rows(m)."""
+    buffer of rows >= tiled_rows(m).  ``tiled``: ``is_tiled(weight)`` where the
+    caller has it."""
     m, k = x.shape
     n = int(weight.shape[0])
     four_wave = m > SKINNY_MAX_M and k >= 256 and n % 8 == 0
     fits = four_wave if lora else (0 < m <= SKINNY_MAX_M or four_wave)
-    if is_tiled(weight) and k % 128 == 0 and fits:
+    if k % 128 == 0 and fits and (is_tiled(weight) if tiled is None else tiled):
         buf = None if codes is None else codes[:tiled_rows(m)]
         q, s = quant_rows_tiled(x, fmt, rounding, codes=buf, scales=scales)
         return q, s, True
@@ -297,6 +325,9 @@ def quant_rows_tiled(x: torch.Tensor, fmt: int, rounding: int = ROUND_DIV, *, co
     dtype with R a multiple of 16 (allocated here as [tiled_rows(rows), K]
     when omitted, which requires row0 == 0).  Scales are returned for the
     quantized rows only ([rows, 1] fp32)."""
+    got = _native_call("quant_rows_tiled", x, fmt, rounding, codes, row0, scales)
+    if got is not None:
+        return got
     _require_gpu("quant_rows_tiled", x, codes, scales)
     _rows_2d("quant_rows_tiled x", x, torch.bfloat16)
     rows, cols = x.shape
@@ -334,11 +365,15 @@ def quant_tensor_e4m3(x: torch.Tensor, static_scale: torch.Tensor | None = None,
     divisor and the quotient are rounded to that dtype, for fp32 neither);
     otherwise the reference's Triton form, the fp32-divisor quotient rounded
     to bf16.  For bf16 input ``bf16_divisor`` is the older name of ``eager``."""
+    if eager is None:
+        eager = bf16_divisor
+    if codes is None and scale is None and workspace is None:
+        got = _native_call("quant_tensor", x, static_scale, bool(eager))
+        if got is not None:
+            return got
     _require_gpu("quant_tensor_e4m3", x, static_scale, codes, scale, workspace)
     if x.dtype not in _TENSOR_DTYPES:
         raise TypeError(f"quant_tensor_e4m3: expected bfloat16, float16 or float32 input, got {x.dtype}")
-    if eager is None:
-        eager = bf16_divisor
     shape = tuple(x.shape)
     x2 = x.reshape(-1, shape[-1]) if x.ndim != 2 else x
     if x2.ndim != 2 or x2.stride(-1) != 1:
@@ -374,6 +409,10 @@ def swiglu_quant(x: torch.Tensor, *, fmt: int | None = None, rounding: int = ROU
     y = bf16(bf16(gate / (1 + exp(-gate))) * up), to ``out`` (a bf16 tensor,
     True to allocate one, None/False for none) and / or per-token codes in
     ``fmt`` (None: no codes).  Returns (out or None, codes or None, scales or None)."""
+    if codes is None and scales is None and not isinstance(out, torch.Tensor):
+        got = _native_call("swiglu_quant", x, -1 if fmt is None else fmt, rounding, out is True)
+        if got is not None:
+            return got
     want_out = out is True or isinstance(out, torch.Tensor)
     _require_gpu("swiglu_quant", x, out if isinstance(out, torch.Tensor) else None, codes, scales)
     _rows_2d("swiglu_quant x", x, torch.bfloat16)
@@ -414,6 +453,10 @@ def quant_per_head_e4m3(x: torch.Tensor, *, codes: torch.Tensor | None = None, s
     """Per-(batch, head) e4m3fn of a bf16 ``x [B, S, H, D]``: (codes [B, S, H, D]
     float8_e4m3fn, scales [B, H] fp32) with scale = max(amax * RN(1/448), 1e-12)
     over (S, D) and an fp32 quotient."""
+    if codes is None and scales is None and workspace is None:
+        got = _native_call("quant_per_head", x)
+        if got is not None:
+            return got
     _require_gpu("quant_per_head_e4m3", x, codes, scales, workspace)
     if x.dtype != torch.bfloat16:
         raise TypeError(f"quant_per_head_e4m3: expected bfloat16 input, got {x.dtype}")
@@ -464,6 +507,11 @@ def scaled_mm(a: torch.Tensor, b: torch.Tensor, a_scale: torch.Tensor, b_scale: 
     ``b_tiled``, see quant_rows_tiled) is a contiguous [R, k] tensor with R the
     row count rounded up to 16; ``m`` / ``n`` give the logical row counts when
     they differ from R."""
+    if (a_tiled or not is_tiled(a)) and (b_tiled or not is_tiled(b)) and out_dtype in _OUT_F16:
+        got = _native_call("scaled_mm", a, b, a_scale, b_scale, bias, lora_t, lora_b, lora_scale, out, a_tiled, b_tiled,
+                           -1 if m is None else m, -1 if n is None else n, _OUT_F16[out_dtype])
+        if got is not None:
+            return got
     _require_gpu("scaled_mm", a, b, a_scale, b_scale, bias, lora_t, lora_b, out)
     if a.dtype not in _FORMATS or b.dtype != a.dtype:
         raise TypeError(f"scaled_mm: operands must both be e4m3fn or int8, got {a.dtype} and {b.dtype}")
@@ -534,6 +582,9 @@ def gemm_i8_i32(a: torch.Tensor, b: torch.Tensor, *, out: torch.Tensor | None = 
 
 def lora_down(x: torch.Tensor, lora_a: torch.Tensor, *, out: torch.Tensor | None = None) -> torch.Tensor:
     """t = bf16(x @ lora_a^T) for bf16 x [m, k], lora_a [r, k]."""
+    got = _native_call("lora_down", x, lora_a, out)
+    if got is not None:
+        return got
     _require_gpu("lora_down", x, lora_a, out)
     _rows_2d("lora_down x", x, torch.bfloat16)
     _rows_2d("lora_down lora_a", lora_a, torch.bfloat16)

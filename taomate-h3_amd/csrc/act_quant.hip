@@ -113,7 +113,7 @@ __device__ __forceinline__ int img_chunk(int c, int r) { return (c & ~15) | ((c 
 
 template <int FMT, int ROUND, int NV, bool PREFETCH>
 __global__ __launch_bounds__(512) void quant_rows_tiled_img_kernel(const uint16_t* __restrict__ x, int64_t ldx,
-                                                                   int64_t units, int k, uint8_t* __restrict__ q,
+                                                                   int64_t rows, int k, uint8_t* __restrict__ q,
                                                                    int64_t row0, float* __restrict__ scales) {
     extern __shared__ __attribute__((aligned(16))) uint8_t img[];
     const int lane = threadIdx.x & 63;
@@ -121,9 +121,15 @@ __global__ __launch_bounds__(512) void quant_rows_tiled_img_kernel(const uint16_
     const int nvec = k >> 3;
     const int64_t steps = k >> 7;
     const int w = (k + 255) & ~255;  // image row stride
+    const int64_t units = (rows + 7) >> 3;
+    // Row r of unit un; a wave past the last row takes zeros, and neither its
+    // scale nor its codes are stored (they may belong to other rows' calls).
+    auto load = [&](int64_t un, auto& dst) __attribute__((always_inline)) {
+        load_row<NV>(x, ldx, 8 * un + r, 8 * un + r < rows ? nvec : 0, lane, dst);
+    };
     uint4 v[NV], vn[PREFETCH ? NV : 1];
     int64_t u = blockIdx.x;
-    if (u < units) load_row<NV>(x, ldx, 8 * u + r, nvec, lane, v);
+    if (u < units) load(u, v);
     while (u < units) {
         const int64_t row = 8 * u + r;
         uint32_t m = 0;
@@ -137,7 +143,7 @@ __global__ __launch_bounds__(512) void quant_rows_tiled_img_kernel(const uint16_
         const float amax = wave_max(amax_from_packed(m));
         RowQuant<FMT, ROUND> rq;
         rq.init(amax);
-        if (lane == 0) scales[row] = rq.s;
+        if (lane == 0 && row < rows) scales[row] = rq.s;
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
             const int vec = i * 64 + lane;  // codes 8 vec .. 8 vec + 7: chunk vec / 2, half vec % 2
@@ -150,7 +156,7 @@ __global__ __launch_bounds__(512) void quant_rows_tiled_img_kernel(const uint16_
         }
         const int64_t un = u + gridDim.x;
         if constexpr (PREFETCH) {
-            if (un < units) load_row<NV>(x, ldx, 8 * un + r, nvec, lane, vn);
+            if (un < units) load(un, vn);
         }
         __syncthreads();
         // Read-back: slot t = ((s * 2 + h) * 4 + qq) * 8 + rr holds row rr,
@@ -159,7 +165,9 @@ __global__ __launch_bounds__(512) void quant_rows_tiled_img_kernel(const uint16_
         const int half = (int)(((row0 + 8 * u) >> 3) & 1);
         uint8_t* const qb = q + blk * steps * 2048;
         const int slots = k >> 1;  // 8 rows x k bytes / 16
+        const int live = rows - 8 * u < 8 ? (int)(rows - 8 * u) : 8;
         for (int t = threadIdx.x; t < slots; t += 512) {
+            if ((t & 7) >= live) continue;
             const int rr = t & 7, qq = (t >> 3) & 3, h = (t >> 5) & 1, s = t >> 6;
             const int c = 8 * s + 2 * qq + h;
             const uint4 val = *reinterpret_cast<const uint4*>(img + rr * w + img_chunk(c, rr) * 16);
@@ -170,7 +178,7 @@ __global__ __launch_bounds__(512) void quant_rows_tiled_img_kernel(const uint16_
 #pragma unroll
             for (int i = 0; i < NV; ++i) v[i] = vn[i];
         } else if (un < units) {
-            load_row<NV>(x, ldx, 8 * un + r, nvec, lane, v);
+            load(un, v);
         }
         u = un;
     }
@@ -214,9 +222,9 @@ static hipError_t launch_rows_vec(const uint16_t* x, int64_t ldx, int64_t rows, 
 }
 
 template <int FMT, int ROUND, int NV, bool PREFETCH>
-static hipError_t launch_rows_tiled_img_cfg(const uint16_t* x, int64_t ldx, int64_t blocks, int64_t k, uint8_t* q,
+static hipError_t launch_rows_tiled_img_cfg(const uint16_t* x, int64_t ldx, int64_t rows, int64_t k, uint8_t* q,
                                             int64_t row0, float* scales, int per_cu, hipStream_t st) {
-    const int64_t units = blocks * 2;
+    const int64_t units = (rows + 7) / 8;
     const int64_t img_bytes = 8 * ((k + 255) & ~int64_t(255));
     const int64_t cap = 256 * (int64_t)per_cu;
     const int64_t grid = units < cap ? units : cap;
@@ -226,34 +234,34 @@ static hipError_t launch_rows_tiled_img_cfg(const uint16_t* x, int64_t ldx, int6
         hipFuncAttributeMaxDynamicSharedMemorySize, 8 * ((512 * NV + 255) & ~255));
     if (lds_limit != hipSuccess) return lds_limit;
     hipLaunchKernelGGL((quant_rows_tiled_img_kernel<FMT, ROUND, NV, PREFETCH>), dim3((unsigned)grid), dim3(512),
-                       (size_t)img_bytes, st, x, ldx, units, (int)k, q, row0, scales);
+                       (size_t)img_bytes, st, x, ldx, rows, (int)k, q, row0, scales);
     return hipGetLastError();
 }
 
 template <int FMT, int ROUND, int NV>
-static hipError_t launch_rows_tiled_img(const uint16_t* x, int64_t ldx, int64_t blocks, int64_t k, uint8_t* q,
+static hipError_t launch_rows_tiled_img(const uint16_t* x, int64_t ldx, int64_t rows, int64_t k, uint8_t* q,
                                         int64_t row0, float* scales, hipStream_t st) {
     // Workgroups of 8 waves: two per CU while the image (8 W bytes) and two
     // row register sets per lane (128 VGPRs) fit twice, else one.
     const int64_t img_bytes = 8 * ((k + 255) & ~int64_t(255));
     const int per_cu = (NV <= 12 && img_bytes <= 80 * 1024) ? 2 : 1;
-    return launch_rows_tiled_img_cfg<FMT, ROUND, NV, true>(x, ldx, blocks, k, q, row0, scales, per_cu, st);
+    return launch_rows_tiled_img_cfg<FMT, ROUND, NV, true>(x, ldx, rows, k, q, row0, scales, per_cu, st);
 }
 
 template <int FMT, int ROUND>
-static hipError_t dispatch_rows_tiled_img(const uint16_t* x, int64_t ldx, int64_t blocks, int64_t k, uint8_t* q,
+static hipError_t dispatch_rows_tiled_img(const uint16_t* x, int64_t ldx, int64_t rows, int64_t k, uint8_t* q,
                                             int64_t row0, float* scales, hipStream_t st) {
     const int64_t nv = (k + 511) / 512;
-    if (nv <= 2) return launch_rows_tiled_img<FMT, ROUND, 2>(x, ldx, blocks, k, q, row0, scales, st);
-    if (nv <= 4) return launch_rows_tiled_img<FMT, ROUND, 4>(x, ldx, blocks, k, q, row0, scales, st);
-    if (nv <= 8) return launch_rows_tiled_img<FMT, ROUND, 8>(x, ldx, blocks, k, q, row0, scales, st);
-    if (nv <= 10) return launch_rows_tiled_img<FMT, ROUND, 10>(x, ldx, blocks, k, q, row0, scales, st);
-    if (nv <= 11) return launch_rows_tiled_img<FMT, ROUND, 11>(x, ldx, blocks, k, q, row0, scales, st);
-    if (nv <= 14) return launch_rows_tiled_img<FMT, ROUND, 14>(x, ldx, blocks, k, q, row0, scales, st);
-    if (nv <= 16) return launch_rows_tiled_img<FMT, ROUND, 16>(x, ldx, blocks, k, q, row0, scales, st);
-    if (nv <= 24) return launch_rows_tiled_img<FMT, ROUND, 24>(x, ldx, blocks, k, q, row0, scales, st);
-    if (nv <= 28) return launch_rows_tiled_img<FMT, ROUND, 28>(x, ldx, blocks, k, q, row0, scales, st);
-    return launch_rows_tiled_img<FMT, ROUND, 32>(x, ldx, blocks, k, q, row0, scales, st);
+    if (nv <= 2) return launch_rows_tiled_img<FMT, ROUND, 2>(x, ldx, rows, k, q, row0, scales, st);
+    if (nv <= 4) return launch_rows_tiled_img<FMT, ROUND, 4>(x, ldx, rows, k, q, row0, scales, st);
+    if (nv <= 8) return launch_rows_tiled_img<FMT, ROUND, 8>(x, ldx, rows, k, q, row0, scales, st);
+    if (nv <= 10) return launch_rows_tiled_img<FMT, ROUND, 10>(x, ldx, rows, k, q, row0, scales, st);
+    if (nv <= 11) return launch_rows_tiled_img<FMT, ROUND, 11>(x, ldx, rows, k, q, row0, scales, st);
+    if (nv <= 14) return launch_rows_tiled_img<FMT, ROUND, 14>(x, ldx, rows, k, q, row0, scales, st);
+    if (nv <= 16) return launch_rows_tiled_img<FMT, ROUND, 16>(x, ldx, rows, k, q, row0, scales, st);
+    if (nv <= 24) return launch_rows_tiled_img<FMT, ROUND, 24>(x, ldx, rows, k, q, row0, scales, st);
+    if (nv <= 28) return launch_rows_tiled_img<FMT, ROUND, 28>(x, ldx, rows, k, q, row0, scales, st);
+    return launch_rows_tiled_img<FMT, ROUND, 32>(x, ldx, rows, k, q, row0, scales, st);
 }
 
 template <int FMT, int ROUND, bool TILED>
@@ -262,18 +270,13 @@ static hipError_t dispatch_rows(const uint16_t* x, int64_t ldx, int64_t rows, in
     const bool aligned = (k % 8 == 0) && (ldx % 8 == 0) && (TILED || ldq % 8 == 0) &&
                          ((uintptr_t)x % 16 == 0) && ((uintptr_t)q % 8 == 0);
     const int64_t nv = (k + 511) / 512;
-    // Tiled output from a block boundary: whole 16-row blocks by the image
-    // kernel (16-byte aligned codes), the remaining rows below.
+    // Tiled output from a block boundary (16-byte aligned codes): the image
+    // kernel, ragged last unit included (a second launch for the rows past the
+    // last whole block took 4 us more at any ragged M); fewer than 16 rows and
+    // other starts below.
     if constexpr (TILED) {
-        if (aligned && nv <= 32 && row0 % 16 == 0 && rows >= 16 && (uintptr_t)q % 16 == 0) {
-            const int64_t blocks = rows / 16;
-            hipError_t e = dispatch_rows_tiled_img<FMT, ROUND>(x, ldx, blocks, k, q, row0, scales, st);
-            if (e != hipSuccess || rows == 16 * blocks) return e;
-            x += 16 * blocks * ldx;
-            scales += 16 * blocks;
-            row0 += 16 * blocks;
-            rows -= 16 * blocks;
-        }
+        if (aligned && nv <= 32 && row0 % 16 == 0 && rows >= 16 && (uintptr_t)q % 16 == 0)
+            return dispatch_rows_tiled_img<FMT, ROUND>(x, ldx, rows, k, q, row0, scales, st);
     }
     if (aligned) {
         if (nv <= 2) return launch_rows_vec<FMT, ROUND, 2, TILED>(x, ldx, rows, k, q, ldq, row0, scales, st);

@@ -329,3 +329,25 @@ def test_int8_rcp_known_answers(ops, device):
         assert (q[r, 0], q[r, 3]) == (127, -127)
         assert s[r] == np.float32(float(E.int8_scale(amax)))
     assert s[-1] == 0.0 and not q[-1].any()
+
+
+@pytest.mark.parametrize("rows", [16, 17, 23, 24, 25, 39, 130])
+@pytest.mark.parametrize("k", [128, 5376])
+def test_tiled_ragged_rows_write_only_their_own(ops, oracle, device, rows, k):
+    """A ragged last unit of the tiled quantizer: its rows' codes and scales
+    are the oracle's and nothing past them is written."""
+    from _util import from_tiled
+
+    print(f"tiled ragged {rows}x{k}", flush=True)
+    x = activations(rows, k, seed=rows + k)
+    total = (rows + 15) // 16 * 16 + 16
+    codes = torch.full((total, k), 77, device=device, dtype=torch.int8)
+    scales = torch.full((rows + 9,), -1.0, device=device)
+    ops.quant_rows_tiled(x.to(device), ops.FMT_INT8, ops.ROUND_RCP_MUL, codes=codes, scales=scales[:rows])
+    torch.cuda.synchronize()
+    rq, rs = oracle.quant_rows(bits16(x), "int8", "rcp")
+    got = from_tiled(bits8(codes), total, k)
+    np.testing.assert_array_equal(got[:rows], rq.view(np.uint8))
+    assert (got[rows:] == 77).all()
+    np.testing.assert_array_equal(scales[:rows].cpu().numpy(), rs)
+    assert (scales[rows:] == -1.0).all()

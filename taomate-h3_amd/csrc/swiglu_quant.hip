@@ -23,8 +23,8 @@
 // where its own exp (the library's, or Triton's) moves the binary32 silu
 // across a bf16 rounding boundary.
 //
-// One wavefront per row, y kept in VGPRs (NV 8-element vectors per lane) for
-// the quantizer; gate and up are read in batches of four vectors per lane.
+// Several waves share a row, y kept in VGPRs (8-element vectors) for the
+// quantizer, so that even a few rows spread over the chip.
 // Per row 4F bytes in, F bytes of codes + 4 bytes of scale out (+ 2F with out).
 //
 // Table form (swiglu_quant_lut_kernel, calls of at least kLutMinRows rows).
@@ -78,23 +78,27 @@ __global__ __launch_bounds__(256) void silu_table_kernel(uint16_t* __restrict__ 
     reinterpret_cast<uint32_t*>(table)[g >> 1] = pack_bf16x2(silu_f32(bf16_lo(w)), silu_f32(bf16_hi(w)));
 }
 
+// Direct form: a workgroup of four waves per row, NV vectors per lane each: wave w
+// takes vectors (4 i + w) * 64 + lane, and the row's maximum is exchanged through
+// LDS (double-buffered by row parity, so one barrier a row).
 template <int FMT, int ROUND, int NV>
 __global__ __launch_bounds__(256) void swiglu_quant_kernel(SwigluQuantArgs p) {
-    const int lane = threadIdx.x & 63;
+    __shared__ uint32_t red[2][4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int nvec = p.half >> 3;
-    const int64_t step = (int64_t)gridDim.x * 4;
-    for (int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); row < p.rows; row += step) {
+    int parity = 0;
+    for (int64_t row = blockIdx.x; row < p.rows; row += gridDim.x) {
         const uint4* gr = reinterpret_cast<const uint4*>(p.x + row * p.ldx);
         const uint4* ur = reinterpret_cast<const uint4*>(p.x + row * p.ldx + p.half);
         uint4 y[NV];
         uint32_t m = 0;
-        constexpr int B = 4;
+        constexpr int B = NV < 4 ? NV : 4;
 #pragma unroll
         for (int i0 = 0; i0 < NV; i0 += B) {
             uint4 g[B], u[B];
 #pragma unroll
             for (int b = 0; b < B; ++b) {
-                const int vec = (i0 + b) * 64 + lane;
+                const int vec = ((i0 + b) * 4 + wave) * 64 + lane;
                 const bool in = i0 + b < NV && vec < nvec;
                 g[b] = in ? gr[vec] : make_uint4(0, 0, 0, 0);
                 u[b] = in ? ur[vec] : make_uint4(0, 0, 0, 0);
@@ -117,16 +121,24 @@ __global__ __launch_bounds__(256) void swiglu_quant_kernel(SwigluQuantArgs p) {
         if (p.out) {
             uint4* orow = reinterpret_cast<uint4*>(p.out + row * p.ldo);
 #pragma unroll
-            for (int i = 0; i < NV; ++i)
-                if (i * 64 + lane < nvec) orow[i * 64 + lane] = y[i];
+            for (int i = 0; i < NV; ++i) {
+                const int vec = (4 * i + wave) * 64 + lane;
+                if (vec < nvec) orow[vec] = y[i];
+            }
         }
         if (p.codes == nullptr) continue;
-        const float amax = wave_max(amax_from_packed(m));
+        const float mine = wave_max(amax_from_packed(m));
+        if (lane == 0) red[parity][wave] = __float_as_uint(mine);
+        __syncthreads();
+        float amax = 0.0f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) amax = mag_max(amax, __uint_as_float(red[parity][w]));
+        parity ^= 1;
         RowQuant<FMT, ROUND> rq;
         rq.init(amax);
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
-            const int vec = i * 64 + lane;
+            const int vec = (4 * i + wave) * 64 + lane;
             if (vec < nvec) {
                 uint2 o;
                 o.x = rq.pack4(y[i].x, y[i].y);
@@ -134,76 +146,100 @@ __global__ __launch_bounds__(256) void swiglu_quant_kernel(SwigluQuantArgs p) {
                 *reinterpret_cast<uint2*>(p.codes + row * p.ldq + 8 * (int64_t)vec) = o;
             }
         }
-        if (lane == 0) p.scales[row] = rq.s;
+        if (threadIdx.x == 0) p.scales[row] = rq.s;
     }
 }
 
-// Table form: one workgroup of LUT_WAVES waves per CU (the 128 KiB table
-// fills most of the LDS), rows dealt to waves in order as above.
-constexpr int kLutWaves = 8;
-template <int FMT, int ROUND, int NV>
+// Table form: one workgroup of 16 waves per CU (the 128 KiB table fills most of
+// the LDS), SPLIT waves to a row, so a workgroup takes groups of 16 / SPLIT rows
+// blockIdx.x, blockIdx.x + grid, ...  The next group's gate and up are requested
+// before the barrier that exchanges this group's maxima, so reads and stores
+// overlap.  Measured on MI355X (int8 codes, inputs rotated, us; a wave per row as
+// before -> this): 2640 x 7168 26.4 -> 22.3, 8192 x 7168 59.6 -> 53.9, 8192 x 13824
+// 119.4 -> 108.4 (5.2 TB/s, the rate of a large copy), 4000 x 14336 58.9 -> 54.5.
+constexpr int kLutWaves = 16;
+template <int FMT, int ROUND, int NV, int SPLIT>
 __global__ __launch_bounds__(kLutWaves * 64) void swiglu_quant_lut_kernel(SwigluQuantArgs p,
                                                                          const uint16_t* __restrict__ table) {
     __shared__ __attribute__((aligned(1024))) uint16_t lds_table[65536];
+    __shared__ uint32_t red[2][kLutWaves];
+    constexpr int kRows = kLutWaves / SPLIT;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int part = wave % SPLIT, sub = wave / SPLIT;
+    const int nvec = p.half >> 3;
+    const int64_t groups = (p.rows + kRows - 1) / kRows;
+    uint4 g[NV], u[NV];
+    auto load = [&](int64_t group) __attribute__((always_inline)) {
+        const int64_t row = group * kRows + sub;
+        if (row >= p.rows) return;
+        const uint4* gr = reinterpret_cast<const uint4*>(p.x + row * p.ldx);
+        const uint4* ur = reinterpret_cast<const uint4*>(p.x + row * p.ldx + p.half);
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const int vec = (i * SPLIT + part) * 64 + lane;
+            if (vec < nvec) {
+                g[i] = gr[vec];
+                u[i] = ur[vec];
+            }
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < NV; ++i) g[i] = u[i] = make_uint4(0, 0, 0, 0);  // lanes past the row: y = 0
     {
-        // 128 KiB by LDS-DMA: 128 wave copies of 1 KiB, 16 per wave.
+        // 128 KiB by LDS-DMA: 128 wave copies of 1 KiB.
         const CopySrc src(table, 65536u * 2u);
-        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
         const uint32_t base = (uint32_t)(uintptr_t)(H3Q_LDS uint16_t*)lds_table;
 #pragma unroll
         for (int i = 0; i < 128 / kLutWaves; ++i) {
             const int c = wave + kLutWaves * i;
             copy16(src, base + (uint32_t)(c * 1024), (uint32_t)(c * 1024 + 16 * lane));
         }
+        load(blockIdx.x);
         wait_vmcnt0();
         __syncthreads();
     }
     const H3Q_LDS uint16_t* t = (const H3Q_LDS uint16_t*)lds_table;
-    const int lane = threadIdx.x & 63;
-    const int nvec = p.half >> 3;
-    const int64_t step = (int64_t)gridDim.x * kLutWaves;
-    for (int64_t row = (int64_t)blockIdx.x * kLutWaves + (threadIdx.x >> 6); row < p.rows; row += step) {
-        const uint4* gr = reinterpret_cast<const uint4*>(p.x + row * p.ldx);
-        const uint4* ur = reinterpret_cast<const uint4*>(p.x + row * p.ldx + p.half);
+    int parity = 0;
+    for (int64_t group = blockIdx.x; group < groups; group += gridDim.x) {
+        const int64_t row = group * kRows + sub;
         uint4 y[NV];
         uint32_t m = 0;
-        constexpr int B = 4;
 #pragma unroll
-        for (int i0 = 0; i0 < NV; i0 += B) {
-            uint4 g[B], u[B];
-#pragma unroll
-            for (int b = 0; b < B; ++b) {
-                const int vec = (i0 + b) * 64 + lane;
-                const bool in = i0 + b < NV && vec < nvec;
-                g[b] = in ? gr[vec] : make_uint4(0, 0, 0, 0);
-                u[b] = in ? ur[vec] : make_uint4(0, 0, 0, 0);
-            }
-#pragma unroll
-            for (int b = 0; b < B; ++b) {
-                if (i0 + b >= NV) break;
-                y[i0 + b] = make_uint4(swiglu2_lut(t, g[b].x, u[b].x), swiglu2_lut(t, g[b].y, u[b].y),
-                                       swiglu2_lut(t, g[b].z, u[b].z), swiglu2_lut(t, g[b].w, u[b].w));
-                // as above: keeps the compiler from holding many vectors' lookups live at once
-                asm volatile("" : "+v"(y[i0 + b].x), "+v"(y[i0 + b].y), "+v"(y[i0 + b].z), "+v"(y[i0 + b].w));
-                m = pk_abs_max(m, y[i0 + b].x);
-                m = pk_abs_max(m, y[i0 + b].y);
-                m = pk_abs_max(m, y[i0 + b].z);
-                m = pk_abs_max(m, y[i0 + b].w);
-            }
+        for (int i = 0; i < NV; ++i) {
+            y[i] = make_uint4(swiglu2_lut(t, g[i].x, u[i].x), swiglu2_lut(t, g[i].y, u[i].y),
+                              swiglu2_lut(t, g[i].z, u[i].z), swiglu2_lut(t, g[i].w, u[i].w));
+            // keeps the compiler from holding many vectors' lookups live at once
+            asm volatile("" : "+v"(y[i].x), "+v"(y[i].y), "+v"(y[i].z), "+v"(y[i].w));
+            m = pk_abs_max(m, y[i].x);
+            m = pk_abs_max(m, y[i].y);
+            m = pk_abs_max(m, y[i].z);
+            m = pk_abs_max(m, y[i].w);
         }
+        load(group + gridDim.x);
+        const float mine = wave_max(amax_from_packed(m));
+        if (lane == 0) red[parity][wave] = __float_as_uint(mine);
+        // (not __syncthreads: the next group's loads stay in flight)
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        float amax = 0.0f;
+#pragma unroll
+        for (int w = 0; w < SPLIT; ++w) amax = mag_max(amax, __uint_as_float(red[parity][sub * SPLIT + w]));
+        parity ^= 1;
+        if (row >= p.rows) continue;
         if (p.out) {
             uint4* orow = reinterpret_cast<uint4*>(p.out + row * p.ldo);
 #pragma unroll
-            for (int i = 0; i < NV; ++i)
-                if (i * 64 + lane < nvec) orow[i * 64 + lane] = y[i];
+            for (int i = 0; i < NV; ++i) {
+                const int vec = (i * SPLIT + part) * 64 + lane;
+                if (vec < nvec) orow[vec] = y[i];
+            }
         }
         if (p.codes == nullptr) continue;
-        const float amax = wave_max(amax_from_packed(m));
         RowQuant<FMT, ROUND> rq;
         rq.init(amax);
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
-            const int vec = i * 64 + lane;
+            const int vec = (i * SPLIT + part) * 64 + lane;
             if (vec < nvec) {
                 uint2 o;
                 o.x = rq.pack4(y[i].x, y[i].y);
@@ -211,15 +247,17 @@ __global__ __launch_bounds__(kLutWaves * 64) void swiglu_quant_lut_kernel(Swiglu
                 *reinterpret_cast<uint2*>(p.codes + row * p.ldq + 8 * (int64_t)vec) = o;
             }
         }
-        if (lane == 0) p.scales[row] = rq.s;
+        if (lane == 0 && part == 0) p.scales[row] = rq.s;
     }
 }
 
 namespace {
 
-// Calls of at least this many rows take the table form (below it the
-// table's copy into every workgroup's LDS is not paid back).
-constexpr int64_t kLutMinRows = 1024;
+// Calls of at least this many rows take the table form; below it the table's copy
+// into every workgroup's LDS is not paid back (F = 7168: 128 rows 5.5 us by the
+// table, 4.7 us direct, 300 rows 6.2 / 7.1 us; F = 14336: 7.7 / 6.8 and 9.0 / 10.8 us).
+// A wave per row, the form before, took 10.1 and 11.0 us, 17.3 and 18.0 us.
+constexpr int64_t kLutMinRows = 192;
 
 // The current device's table, filled on first use (launch + wait, once per
 // device), and its CU count; null while a graph is being captured on st and
@@ -265,40 +303,39 @@ hipError_t silu_table_for(hipStream_t st, const uint16_t** out, int* cus) {
     return hipSuccess;
 }
 
-template <int FMT, int ROUND, int NV>
+// ND: vectors per lane of the direct form (four waves a row); NT, SPLIT: those of
+// the table form.
+template <int FMT, int ROUND, int ND, int NT, int SPLIT>
 hipError_t launch_sq_nv(const SwigluQuantArgs& a, hipStream_t st) {
-    // (the widest rows, NV = 32, would spill registers in the table form)
-    if constexpr (NV <= 28) {
-        if (a.rows >= kLutMinRows) {
-            const uint16_t* table = nullptr;
-            int cus = 0;
-            const hipError_t e = silu_table_for(st, &table, &cus);
-            if (e != hipSuccess) return e;
-            if (table) {
-                const int64_t waves = (a.rows + kLutWaves - 1) / kLutWaves;
-                const int64_t blocks = waves < cus ? waves : cus;
-                hipLaunchKernelGGL((swiglu_quant_lut_kernel<FMT, ROUND, NV>), dim3((unsigned)blocks),
-                                   dim3(kLutWaves * 64), 0, st, a, table);
-                return hipGetLastError();
-            }
+    if (a.rows >= kLutMinRows) {
+        const uint16_t* table = nullptr;
+        int cus = 0;
+        const hipError_t e = silu_table_for(st, &table, &cus);
+        if (e != hipSuccess) return e;
+        if (table) {
+            constexpr int kRows = kLutWaves / SPLIT;
+            const int64_t groups = (a.rows + kRows - 1) / kRows;
+            const int64_t blocks = groups < cus ? groups : cus;
+            hipLaunchKernelGGL((swiglu_quant_lut_kernel<FMT, ROUND, NT, SPLIT>), dim3((unsigned)blocks),
+                               dim3(kLutWaves * 64), 0, st, a, table);
+            return hipGetLastError();
         }
     }
-    constexpr int64_t kBlocks = 1024;
-    const int64_t blocks = (a.rows + 3) / 4 < kBlocks ? (a.rows + 3) / 4 : kBlocks;
-    hipLaunchKernelGGL((swiglu_quant_kernel<FMT, ROUND, NV>), dim3((unsigned)blocks), dim3(256), 0, st, a);
+    constexpr int64_t kBlocks = 8192;
+    const int64_t blocks = a.rows < kBlocks ? a.rows : kBlocks;
+    hipLaunchKernelGGL((swiglu_quant_kernel<FMT, ROUND, ND>), dim3((unsigned)blocks), dim3(256), 0, st, a);
     return hipGetLastError();
 }
 
 template <int FMT, int ROUND>
 hipError_t launch_sq_fmt(const SwigluQuantArgs& a, hipStream_t st) {
     const int nvec = a.half / 8;
-    if (nvec <= 128) return launch_sq_nv<FMT, ROUND, 2>(a, st);
-    if (nvec <= 256) return launch_sq_nv<FMT, ROUND, 4>(a, st);
-    if (nvec <= 512) return launch_sq_nv<FMT, ROUND, 8>(a, st);
-    if (nvec <= 1024) return launch_sq_nv<FMT, ROUND, 16>(a, st);
-    if (nvec <= 1728) return launch_sq_nv<FMT, ROUND, 27>(a, st);  // F = 13824 exactly
-    if (nvec <= 1792) return launch_sq_nv<FMT, ROUND, 28>(a, st);
-    return launch_sq_nv<FMT, ROUND, 32>(a, st);
+    if (nvec <= 256) return launch_sq_nv<FMT, ROUND, 1, 1, 4>(a, st);
+    if (nvec <= 512) return launch_sq_nv<FMT, ROUND, 2, 2, 4>(a, st);
+    if (nvec <= 1024) return launch_sq_nv<FMT, ROUND, 4, 2, 8>(a, st);
+    if (nvec <= 1536) return launch_sq_nv<FMT, ROUND, 6, 3, 8>(a, st);
+    if (nvec <= 1792) return launch_sq_nv<FMT, ROUND, 7, 4, 8>(a, st);
+    return launch_sq_nv<FMT, ROUND, 8, 4, 8>(a, st);
 }
 
 }  // namespace

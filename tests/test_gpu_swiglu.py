@@ -195,3 +195,12 @@ def test_host_checks(ops, device):
     with pytest.raises(RuntimeError, match="division form"):
         ops.swiglu_quant(torch.zeros(2, 32, dtype=torch.bfloat16, device=device), fmt=ops.FMT_E4M3FN,
                          rounding=ops.ROUND_RCP_MUL)
+
+
+@pytest.mark.parametrize("fmt,rounding", FMTS)
+@pytest.mark.parametrize("rows,half", [(191, 1024), (192, 1024), (193, 4096), (515, 7168), (195, 8200), (261, 14336),
+                                       (197, 16384), (1, 16384), (33, 4104)])
+def test_swiglu_rows_shared_by_waves(ops, oracle, device, fmt, rounding, rows, half):
+    """Both sides of the row count where the table form starts, ragged last
+    row groups, and row widths at the edges of each number of vectors per lane."""
+    test_swiglu_matches_oracle(ops, oracle, device, fmt, rounding, rows, half)

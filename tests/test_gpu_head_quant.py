@@ -202,3 +202,18 @@ def test_heads_with_infinities_and_nans(ops, oracle, device, shape):
         nan_q = (want & 0x7F) == 0x7F
         np.testing.assert_array_equal((got & 0x7F) == 0x7F, nan_q)
         np.testing.assert_array_equal(np.where(nan_q, 0, got), np.where(nan_q, 0, want))
+
+
+@pytest.mark.parametrize("shape", [(1, 4096, 5, 64), (1, 4097, 5, 64), (2, 3121, 9, 128), (1, 40, 70, 128),
+                                   (2, 1000, 3, 1024), (1, 513, 6, 20)])
+def test_scales_folded_by_the_quantize_pass(ops, oracle, device, shape):
+    """Both sides of the chunk count up to which the quantize pass folds the
+    partial maxima itself; heads that straddle column groups, several batches."""
+    print(f"per-head fold {shape}", flush=True)
+    gen = torch.Generator().manual_seed(sum(shape))
+    x = (torch.randn(shape, generator=gen) * torch.rand(shape[2], 1, generator=gen) * 4).to(torch.bfloat16)
+    codes, scales = ops.quant_per_head_e4m3(x.to(device))
+    torch.cuda.synchronize()
+    rq, rs = oracle.quant_per_head_e4m3(bits16(x).reshape(shape))
+    np.testing.assert_array_equal(bits8(codes).reshape(-1), np.asarray(rq).reshape(-1).view(np.uint8))
+    np.testing.assert_array_equal(scales.cpu().numpy().reshape(-1), np.asarray(rs).reshape(-1))

@@ -26,15 +26,10 @@ hipError_t tensor_scratch(float** out);
 enum TensorIn : int { kInBF16 = 0, kInF16 = 1, kInF32 = 2 };
 
 // Per-tensor e4m3 of bf16 / fp16 / fp32 input; eager: torch's clamp(x / s) in
-// x's dtype, else the fp32-divisor quotient rounded to bf16.  bf16 input runs
-// the vector kernels of launch_quant_tensor_e4m3.
+// x's dtype, else the fp32-divisor quotient rounded to bf16.
 hipError_t launch_quant_tensor_e4m3_typed(const void* x, int in, bool eager, int64_t ldx, int64_t rows, int64_t k,
                                           const float* static_scale, float* partial, uint8_t* q, int64_t ldq,
                                           float* scale_out, hipStream_t st);
-
-hipError_t launch_quant_tensor_e4m3(const uint16_t* x, int64_t ldx, int64_t rows, int64_t k,
-                                    const float* static_scale, bool bf16_divisor, float* partial, uint8_t* q,
-                                    int64_t ldq, float* scale_out, hipStream_t st);
 
 // Fused SwiGLU (+ per-token quantization): rows of x are [gate (half) | up
 // (half)] bf16; y = bf16(bf16(silu(gate)) * up) to out (optional, [rows, half])

@@ -230,3 +230,39 @@ def test_fp8_dynamic_linear_module(oracle, device, monkeypatch, fused):
     rqa, rsa = oracle.quant_tensor_e4m3_typed(_bits(x.reshape(80, 256)), "f16", not fused)
     _assert_fp8_f16_close(oracle, bits16(out.reshape(80, 512)), rqa, np.array([rsa]), rqw, np.array([rsw]),
                           _bits(b0.to(torch.float16)))
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("eager,static", [(False, False), (True, False), (True, True)])
+@pytest.mark.parametrize(
+    "m,k",
+    [
+        (1, 8),        # one vector: lanes and loads past the end
+        (9, 2048),     # nine chunks of 256 vectors: the first grid that is cut to a multiple of 8
+        (3, 2056),     # a last chunk of 3 vectors
+        (2049, 2048),  # 2049 chunks: two per workgroup from here on, the last one almost empty
+        (4099, 2056),  # more than 4096 chunks: four in flight, several trips, a ragged tail
+    ],
+)
+def test_tensor_quant_vectors_match_the_oracle(ops, oracle, device, dtype, eager, static, m, k):
+    """The vector path, rows adjacent and rows 8 elements apart, infinities and a NaN under a
+    static scale (a vector that holds one is redone element by element)."""
+    print(f"tensor vectors {dtype} eager={eager} static={static} {m}x{k}", flush=True)
+    gen = torch.Generator().manual_seed(m + k)
+    x = (torch.randn(m, k, generator=gen) * torch.exp2(torch.randint(-8, 4, (1, k), generator=gen).float()))
+    x = x.to(torch.bfloat16 if dtype == "bf16" else _DT[dtype])
+    if static:
+        x[0, 3], x[-1, -1], x[m // 2, k // 2] = float("inf"), float("-inf"), float("nan")
+    st = 0.0371 if static else None
+    sg = torch.tensor(st, dtype=torch.float32, device=device) if static else None
+    bits = x.view(torch.int16).numpy().view(np.uint16) if dtype == "bf16" else _bits(x)
+    rq, rs = oracle.quant_tensor_e4m3_typed(bits, dtype, eager, st)
+    wide = torch.full((m, k + 8), 7.0e4 if dtype == "f32" else 6.0e4, dtype=x.dtype, device=device)
+    wide[:, :k] = x.to(device)
+    for xd in (x.to(device), wide[:, :k]):
+        q, s = ops.quant_tensor_e4m3(xd, sg, eager=eager)
+        torch.cuda.synchronize()
+        assert np.float32(s.item()) == rs
+        got, nan_q = bits8(q), (rq & 0x7F) == 0x7F
+        np.testing.assert_array_equal((got & 0x7F) == 0x7F, nan_q)
+        np.testing.assert_array_equal(np.where(nan_q, 0, got), np.where(nan_q, 0, rq))

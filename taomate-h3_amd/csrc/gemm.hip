@@ -733,7 +733,10 @@ hipError_t launch_gemm(int kind, bool raw_i32, const GemmArgs& args, hipStream_t
         if (const int tile = stream_tile(a)) return launch_gemm_stream(kind, tile, a, st);
     }
     if (kind != kOpBF16 && !raw_i32 && skinny_supported(a)) return launch_gemm_skinny(kind, a, st);
-    if (kind != kOpBF16 && !raw_i32 && w4_supported(a)) return launch_gemm_w4(kind, a, st);
+    if (kind != kOpBF16 && !raw_i32 && w4_supported(a)) {
+        const GemmSplit split = gemm_split(a);
+        return split.at ? launch_gemm_split(kind, split, a, st) : launch_gemm_w4(kind, a, st);
+    }
     if (kind == kOpE4M3)
         return lora ? launch_scaled<TileBigLora, kOpE4M3, true>(a, st) : launch_scaled<TileBig, kOpE4M3, false>(a, st);
     if (kind == kOpInt8) {

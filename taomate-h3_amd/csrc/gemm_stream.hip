@@ -13,6 +13,8 @@ struct StreamTile {
 constexpr StreamTile kTiles[] = {{42, 64, 64},   {44, 64, 128},  {54, 80, 128}, {64, 96, 128},  {74, 112, 128},
                                  {84, 128, 128}, {58, 80, 256},  {68, 96, 256}, {78, 112, 256}, {88, 128, 256}};
 constexpr int64_t kCus = 256;
+// Predicted time of a split call over that of the four-wave kernel alone, at most.
+constexpr double kSplitGain = 0.98;
 
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
@@ -22,10 +24,31 @@ int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // Fitted to 84 measured calls (N x K of the H3 and benchmark projections, M =
 // 40 .. 3200, tiled operands); it picks the fastest of the ten tiles or one
 // within 6% of it in 80 of them.
-double stream_cost(const StreamTile& t, const GemmArgs& a) {
+double stream_cost(const StreamTile& t, int64_t m, int64_t n, int64_t k) {
     const double per_ktile = 8e-4 * (t.bm + t.bn) + 1.3e-5 * t.bm * t.bn;
-    const int64_t rounds = ceil_div(ceil_div(a.m, t.bm) * ceil_div(a.n, t.bn), kCus);
-    return 2.0 + rounds * (3.5 + a.k / 128.0 * per_ktile);
+    const int64_t rounds = ceil_div(ceil_div(m, t.bm) * ceil_div(n, t.bn), kCus);
+    return 2.0 + rounds * (3.5 + k / 128.0 * per_ktile);
+}
+
+struct StreamChoice {
+    int tile;
+    double cost;
+};
+StreamChoice best_stream_tile(int64_t m, int64_t n, int64_t k) {
+    StreamChoice best{0, 0.0};
+    for (const StreamTile& t : kTiles) {
+        const double c = stream_cost(t, m, n, k);
+        if (best.tile == 0 || c < best.cost) best = {t.id, c};
+    }
+    return best;
+}
+
+// The forms and offsets that gemm_stream_kernel takes.
+bool stream_takes(const GemmArgs& a) {
+    // 16-byte output pieces and 32-bit block-relative offsets.
+    if (a.n % 8 || a.ldo % 8 || (uintptr_t)a.out % 16 || a.k < 128) return false;
+    if (a.lora_t && (a.out_f16 || a.lora_rank > 128)) return false;
+    return 256 * a.k < (int64_t(1) << 30);
 }
 
 // The same of the four-wave kernel: 64-byte k-steps of 0.68 us in a full round
@@ -43,39 +66,89 @@ double four_wave_cost(const GemmArgs& a) {
 // The rule looks at sizes only (never at the layouts when an adapter is
 // present), so a call gives the same bits whatever layout its operands have.
 int stream_tile(const GemmArgs& a) {
-    // 16-byte output pieces and 32-bit block-relative offsets.
-    if (a.n % 8 || a.ldo % 8 || (uintptr_t)a.out % 16 || a.k < 128) return 0;
-    if (a.lora_t && (a.out_f16 || a.lora_rank > 128)) return 0;
-    if (256 * a.k >= (int64_t(1) << 30)) return 0;
-    const StreamTile* best = nullptr;
-    double cost = 0.0;
-    for (const StreamTile& t : kTiles) {
-        const double c = stream_cost(t, a);
-        if (best == nullptr || c < cost) {
-            best = &t;
-            cost = c;
-        }
-    }
+    if (!stream_takes(a)) return 0;
+    const StreamChoice best = best_stream_tile(a.m, a.n, a.k);
     if (a.m > kSkinnyMaxM) {
         // Against the four-wave kernel (or the 16-wave one where K is not a
         // multiple of 128): 0.78 keeps the calls that gain in both weight
         // states (Infinity Cache, HBM) and both layouts; of those left out the
         // best gained 8% in one state and lost 3% in the other.
-        return cost < 0.78 * four_wave_cost(a) ? best->id : 0;
+        return best.cost < 0.78 * four_wave_cost(a) ? best.tile : 0;
     }
     // Against the weight-streaming kernels of M <= 128, which take no adapter.
-    if (a.lora_t) return best->id;  // M = 40, 10752 x 5376, rank 64: 61 us by the per-tile kernel
+    if (a.lora_t) return best.tile;  // M = 40, 10752 x 5376, rank 64: 61 us by the per-tile kernel
     if (a.b_tiled) {
         // They give every CU 32 columns and all of A: 14.8 against 11.8 us at
         // 128 x 5120 x 5120, but 10.8 against 11.8 us at M = 64; above 8192
         // columns their 32-column workgroups no longer fit one round (M = 40,
         // N = 10752: 20.6 against 14.5 us; N = 5120: 10.2 against 11.3 us).
-        return a.m > 64 || (a.m > 32 && a.n > 8192) ? best->id : 0;
+        return a.m > 64 || (a.m > 32 && a.n > 8192) ? best.tile : 0;
     }
     // Row-major weights: 20 x 5120 x 5120 14.0 against 13.2 us, 100 x 5120 x
     // 5120 38 against 14 us; short K the other way (64 x 2048 x 2048 7.4 against
     // 8.1 us, 64 x 1024 x 1040 5.0 against 7.1 us).
-    return (a.m > 16 && a.k >= 3072) || (a.m > 64 && a.k >= 2048) ? best->id : 0;
+    return (a.m > 16 && a.k >= 3072) || (a.m > 64 && a.k >= 2048) ? best.tile : 0;
+}
+
+// A last round of a few 256 x 256 tiles costs the four-wave kernel 0.51 us per
+// 64-byte step on an otherwise idle chip.  Here full rounds keep that kernel (the
+// first columns or rows of the output) and what is left is spread over all CUs by
+// smaller weight-streaming tiles, in a second launch.  The candidates are the
+// largest first part of all full rounds and of one fewer, by columns and by rows.
+// Sizes only, as above.  Measured on 44 calls (1223 .. 19873 rows, H3 and
+// benchmark projections, with the quantizer): predicted below 0.8 of one launch
+// 10-15% faster (3179 x 5376 x 7168 154 -> 133 us, 6411 x 5120 x 13824 444 -> 389),
+// 0.8-0.9 3-8%, 0.9-0.98 0-3% (one of 20 0.1% slower), above it -0.3 .. +1.3%.
+GemmSplit gemm_split(const GemmArgs& a) {
+    GemmSplit split{false, 0, 0};
+    if (!stream_takes(a)) return split;
+    const int64_t tiles_m = ceil_div(a.m, 256), tiles_n = ceil_div(a.n, 256);
+    const int64_t rounds = tiles_m * tiles_n / kCus;
+    if (rounds == 0 || tiles_m * tiles_n % kCus == 0) return split;
+    double cost = kSplitGain * four_wave_cost(a);
+    for (int64_t full = rounds; full > 0 && full >= rounds - 1; --full) {
+        const double main = 8.0 + a.k / 64.0 * 0.68 * full;
+        const int64_t n0 = full * kCus / tiles_m * 256, m0 = full * kCus / tiles_n * 256;
+        if (n0 > 0 && n0 < a.n) {
+            const StreamChoice rest = best_stream_tile(a.m, a.n - n0, a.k);
+            if (main + rest.cost < cost) {
+                split = {true, n0, rest.tile};
+                cost = main + rest.cost;
+            }
+        }
+        if (m0 > 0 && m0 < a.m) {
+            const StreamChoice rest = best_stream_tile(a.m - m0, a.n, a.k);
+            if (main + rest.cost < cost) {
+                split = {false, m0, rest.tile};
+                cost = main + rest.cost;
+            }
+        }
+    }
+    return split;
+}
+
+hipError_t launch_gemm_split(int kind, const GemmSplit& split, const GemmArgs& a, hipStream_t st) {
+    GemmArgs head = a, rest = a;
+    if (split.columns) {
+        const int64_t n0 = split.at;
+        head.n = n0;
+        rest.n = a.n - n0;
+        rest.b = (const uint8_t*)a.b + (a.b_tiled ? n0 / 16 * (a.k / 128) * 2048 : n0 * a.ldb);
+        if (a.b_scale_per_col) rest.b_scale = a.b_scale + n0;
+        if (a.bias) rest.bias = a.bias + n0;
+        if (a.lora_t) rest.lora_b = a.lora_b + n0 * a.ldlb;
+        rest.out = (uint16_t*)a.out + n0;
+    } else {
+        const int64_t m0 = split.at;
+        head.m = m0;
+        rest.m = a.m - m0;
+        rest.a = (const uint8_t*)a.a + (a.a_tiled ? m0 / 16 * (a.k / 128) * 2048 : m0 * a.lda);
+        if (a.a_scale_per_row) rest.a_scale = a.a_scale + m0;
+        if (a.lora_t) rest.lora_t = a.lora_t + m0 * a.ldt;
+        rest.out = (uint16_t*)a.out + m0 * a.ldo;
+    }
+    const hipError_t e = launch_gemm_w4(kind, head, st);
+    return e != hipSuccess ? e : launch_gemm_stream(kind, split.tile, rest, st);
 }
 
 hipError_t launch_gemm_stream(int kind, int tile, const GemmArgs& a, hipStream_t st) {

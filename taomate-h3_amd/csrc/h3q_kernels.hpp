@@ -116,6 +116,17 @@ hipError_t launch_gemm_skinny(int kind, const GemmArgs& a, hipStream_t st);
 int stream_tile(const GemmArgs& a);
 hipError_t launch_gemm_stream(int kind, int tile, const GemmArgs& a, hipStream_t st);
 
+// A call in two launches: its first columns (or rows) in full rounds of the
+// four-wave kernel, the rest over weight-streaming tiles.  at: columns or rows of
+// the first part, a multiple of 256 (0: one launch is the better one).
+struct GemmSplit {
+    bool columns;
+    int64_t at;
+    int tile;
+};
+GemmSplit gemm_split(const GemmArgs& a);
+hipError_t launch_gemm_split(int kind, const GemmSplit& split, const GemmArgs& a, hipStream_t st);
+
 // Fused RMSNorm + AdaLN modulate (+ residual gate) + per-token quantization
 // (norm_quant.hip).  All bf16 tensors are row-major with element strides;
 // tables are [T, table_stride] and row r uses table row indices[r].

@@ -1,9 +1,9 @@
 // Per-row (per-token / per-output-channel) and per-tensor quantization of a
 // bf16 matrix to OCP e4m3fn or int8 codes, gfx950.
 //
-// Row kernel: one wavefront per row.  The whole row stays in VGPRs (NV 16-byte
-// vectors per lane, 64 lanes read 1 KiB contiguous per step), so X is read from
-// HBM exactly once: abs-max over packed bf16 bit patterns (v_pk_max_u16), a
+// Row kernels: a wavefront or a workgroup of four per row.  The whole row stays in
+// VGPRs (NV 16-byte vectors per lane, 64 lanes read 1 KiB contiguous per step), so X
+// is read from HBM exactly once: abs-max over packed bf16 bit patterns (v_pk_max_u16), a
 // butterfly wave reduction, one IEEE reciprocal per row, then a 3-op
 // correctly rounded quotient per element and 8-byte coalesced code stores.
 // Algorithmic traffic: 2*K read + K written + 4 bytes of scale per row.
@@ -32,8 +32,8 @@ __device__ __forceinline__ int64_t code_offset(int64_t row, int64_t k, int64_t l
 }
 
 // Vector path: K % 8 == 0, x rows 16-byte aligned, q rows 8-byte aligned, K <= NV*512.
-// TILED: codes go to the tiled layout at absolute row row0 + row.
-template <int FMT, int ROUND, int NV, bool TILED>
+// Codes go to the tiled layout at absolute row row0 + row, a wave per row.
+template <int FMT, int ROUND, int NV>
 __global__ __launch_bounds__(256) void quant_rows_vec_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                              int64_t rows, int k, uint8_t* __restrict__ q,
                                                              int64_t ldq, int64_t row0,
@@ -70,10 +70,57 @@ __global__ __launch_bounds__(256) void quant_rows_vec_kernel(const uint16_t* __r
                 uint2 out;
                 out.x = rq.pack4(v[i].x, v[i].y);
                 out.y = rq.pack4(v[i].z, v[i].w);
-                *reinterpret_cast<uint2*>(q + code_offset<TILED>(row0 + row, 8 * (int64_t)vec, ldq)) = out;
+                *reinterpret_cast<uint2*>(q + code_offset<true>(row0 + row, 8 * (int64_t)vec, ldq)) = out;
             }
         }
         if (lane == 0) scales[row] = rq.s;
+    }
+}
+
+// Row-major codes, and tiled codes of few rows: a workgroup of four waves per
+// row, NV vectors per thread (K <= NV * 2048), so that a quarter of the row's loads
+// and conversions stands in each wave's chain and rows in flight fill the chip at
+// a quarter of the registers.  Same alignment; TILED as above.
+template <int FMT, int ROUND, int NV, bool TILED>
+__global__ __launch_bounds__(256) void quant_rows_wide_kernel(const uint16_t* __restrict__ x, int64_t ldx,
+                                                              int64_t rows, int k, uint8_t* __restrict__ q,
+                                                              int64_t ldq, int64_t row0,
+                                                              float* __restrict__ scales) {
+    __shared__ float red[2][4];  // by parity of the row: one barrier per row
+    const int nvec = k >> 3;
+    int par = 0;
+    for (int64_t row = blockIdx.x; row < rows; row += gridDim.x, par ^= 1) {
+        const uint4* xr = reinterpret_cast<const uint4*>(x + row * ldx);
+        uint4 v[NV];
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const int vec = i * 256 + (int)threadIdx.x;
+            v[i] = xr[vec < nvec ? vec : nvec - 1];  // past the end: the last vector again
+        }
+        uint32_t m = 0;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            m = pk_abs_max(m, v[i].x);
+            m = pk_abs_max(m, v[i].y);
+            m = pk_abs_max(m, v[i].z);
+            m = pk_abs_max(m, v[i].w);
+        }
+        const float w = wave_max(amax_from_packed(m));
+        if ((threadIdx.x & 63) == 0) red[par][threadIdx.x >> 6] = w;
+        __syncthreads();
+        RowQuant<FMT, ROUND> rq;
+        rq.init(mag_max(mag_max(red[par][0], red[par][1]), mag_max(red[par][2], red[par][3])));
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const int vec = i * 256 + (int)threadIdx.x;
+            if (vec < nvec) {
+                uint2 out;
+                out.x = rq.pack4(v[i].x, v[i].y);
+                out.y = rq.pack4(v[i].z, v[i].w);
+                *reinterpret_cast<uint2*>(q + code_offset<TILED>(row0 + row, 8 * (int64_t)vec, ldq)) = out;
+            }
+        }
+        if (threadIdx.x == 0) scales[row] = rq.s;
     }
 }
 
@@ -209,14 +256,30 @@ __global__ __launch_bounds__(256) void quant_rows_any_kernel(const uint16_t* __r
 }
 
 constexpr int64_t kRowBlocks = 1024;
+constexpr int64_t kWideBlocks = 1 << 20;
+// Tiled codes up to which a workgroup per row is faster than the 8-row image,
+// whose one unit per CU serializes load, conversion and store: 16 x 5120 4.9 against
+// 2.9 us, 77 x 5376 6.1 / 3.1, 200 x 7168 6.4 / 3.9, 400 x 14336 12.0 / 7.8; even at 800 rows
+// (K = 5120 6.2 / 6.2, 7168 7.9 / 7.5, 14336 13.3 / 13.8), where its 8-byte stores into
+// 16-row blocks begin to cost (1600 x 5120 8.2 / 9.6).
+constexpr int64_t kWideTiledRows = 600;
 
-template <int FMT, int ROUND, int NV, bool TILED>
+template <int FMT, int ROUND, int NV>
 static hipError_t launch_rows_vec(const uint16_t* x, int64_t ldx, int64_t rows, int64_t k, uint8_t* q,
                                   int64_t ldq, int64_t row0, float* scales, hipStream_t st) {
     // One wave per row up to 4 waves per SIMD of the chip (1024 workgroups of
     // four waves on 256 CUs); beyond that each wave takes several rows.
     const int64_t blocks = (rows + 3) / 4 < kRowBlocks ? (rows + 3) / 4 : kRowBlocks;
-    hipLaunchKernelGGL((quant_rows_vec_kernel<FMT, ROUND, NV, TILED>), dim3((unsigned)blocks), dim3(256), 0, st, x,
+    hipLaunchKernelGGL((quant_rows_vec_kernel<FMT, ROUND, NV>), dim3((unsigned)blocks), dim3(256), 0, st, x,
+                       ldx, rows, (int)k, q, ldq, row0, scales);
+    return hipGetLastError();
+}
+
+template <int FMT, int ROUND, int NV, bool TILED>
+static hipError_t launch_rows_wide(const uint16_t* x, int64_t ldx, int64_t rows, int64_t k, uint8_t* q, int64_t ldq,
+                                   int64_t row0, float* scales, hipStream_t st) {
+    const int64_t blocks = rows < kWideBlocks ? rows : kWideBlocks;
+    hipLaunchKernelGGL((quant_rows_wide_kernel<FMT, ROUND, NV, TILED>), dim3((unsigned)blocks), dim3(256), 0, st, x,
                        ldx, rows, (int)k, q, ldq, row0, scales);
     return hipGetLastError();
 }
@@ -270,27 +333,36 @@ static hipError_t dispatch_rows(const uint16_t* x, int64_t ldx, int64_t rows, in
     const bool aligned = (k % 8 == 0) && (ldx % 8 == 0) && (TILED || ldq % 8 == 0) &&
                          ((uintptr_t)x % 16 == 0) && ((uintptr_t)q % 8 == 0);
     const int64_t nv = (k + 511) / 512;
+    // Row-major: always the workgroup per row; a wave per row measured 3.6 against 2.8
+    // us at 16 x 5120, 8.4 / 5.2 at 400 x 14336, 11.7 / 9.5 at 3200 x 5120, 202 / 192 at
+    // 24576 x 14336.
+    if (aligned && nv <= 32 && (!TILED || rows <= kWideTiledRows)) {
+        if (nv <= 4) return launch_rows_wide<FMT, ROUND, 1, TILED>(x, ldx, rows, k, q, ldq, row0, scales, st);
+        if (nv <= 8) return launch_rows_wide<FMT, ROUND, 2, TILED>(x, ldx, rows, k, q, ldq, row0, scales, st);
+        if (nv <= 12) return launch_rows_wide<FMT, ROUND, 3, TILED>(x, ldx, rows, k, q, ldq, row0, scales, st);
+        if (nv <= 16) return launch_rows_wide<FMT, ROUND, 4, TILED>(x, ldx, rows, k, q, ldq, row0, scales, st);
+        if (nv <= 28) return launch_rows_wide<FMT, ROUND, 7, TILED>(x, ldx, rows, k, q, ldq, row0, scales, st);
+        return launch_rows_wide<FMT, ROUND, 8, TILED>(x, ldx, rows, k, q, ldq, row0, scales, st);
+    }
     // Tiled output from a block boundary (16-byte aligned codes): the image
     // kernel, ragged last unit included (a second launch for the rows past the
-    // last whole block took 4 us more at any ragged M); fewer than 16 rows and
-    // other starts below.
+    // last whole block took 4 us more at any ragged M); other starts by a wave per row
+    // (6000 x 14336 87 us; a workgroup per row 97).
     if constexpr (TILED) {
-        if (aligned && nv <= 32 && row0 % 16 == 0 && rows >= 16 && (uintptr_t)q % 16 == 0)
+        if (aligned && nv <= 32 && row0 % 16 == 0 && (uintptr_t)q % 16 == 0)
             return dispatch_rows_tiled_img<FMT, ROUND>(x, ldx, rows, k, q, row0, scales, st);
-    }
-    if (aligned) {
-        if (nv <= 2) return launch_rows_vec<FMT, ROUND, 2, TILED>(x, ldx, rows, k, q, ldq, row0, scales, st);
-        if (nv <= 4) return launch_rows_vec<FMT, ROUND, 4, TILED>(x, ldx, rows, k, q, ldq, row0, scales, st);
-        // nv = 16-byte vectors per lane (512 columns each); exact sizes for the H3
-        // and benchmark widths (K = 5120, 5376, 7168, 13824) keep no idle vectors.
-        if (nv <= 8) return launch_rows_vec<FMT, ROUND, 8, TILED>(x, ldx, rows, k, q, ldq, row0, scales, st);
-        if (nv <= 10) return launch_rows_vec<FMT, ROUND, 10, TILED>(x, ldx, rows, k, q, ldq, row0, scales, st);
-        if (nv <= 11) return launch_rows_vec<FMT, ROUND, 11, TILED>(x, ldx, rows, k, q, ldq, row0, scales, st);
-        if (nv <= 14) return launch_rows_vec<FMT, ROUND, 14, TILED>(x, ldx, rows, k, q, ldq, row0, scales, st);
-        if (nv <= 16) return launch_rows_vec<FMT, ROUND, 16, TILED>(x, ldx, rows, k, q, ldq, row0, scales, st);
-        if (nv <= 24) return launch_rows_vec<FMT, ROUND, 24, TILED>(x, ldx, rows, k, q, ldq, row0, scales, st);
-        if (nv <= 28) return launch_rows_vec<FMT, ROUND, 28, TILED>(x, ldx, rows, k, q, ldq, row0, scales, st);
-        if (nv <= 32) return launch_rows_vec<FMT, ROUND, 32, TILED>(x, ldx, rows, k, q, ldq, row0, scales, st);
+        if (aligned) {
+            if (nv <= 2) return launch_rows_vec<FMT, ROUND, 2>(x, ldx, rows, k, q, ldq, row0, scales, st);
+            if (nv <= 4) return launch_rows_vec<FMT, ROUND, 4>(x, ldx, rows, k, q, ldq, row0, scales, st);
+            if (nv <= 8) return launch_rows_vec<FMT, ROUND, 8>(x, ldx, rows, k, q, ldq, row0, scales, st);
+            if (nv <= 10) return launch_rows_vec<FMT, ROUND, 10>(x, ldx, rows, k, q, ldq, row0, scales, st);
+            if (nv <= 11) return launch_rows_vec<FMT, ROUND, 11>(x, ldx, rows, k, q, ldq, row0, scales, st);
+            if (nv <= 14) return launch_rows_vec<FMT, ROUND, 14>(x, ldx, rows, k, q, ldq, row0, scales, st);
+            if (nv <= 16) return launch_rows_vec<FMT, ROUND, 16>(x, ldx, rows, k, q, ldq, row0, scales, st);
+            if (nv <= 24) return launch_rows_vec<FMT, ROUND, 24>(x, ldx, rows, k, q, ldq, row0, scales, st);
+            if (nv <= 28) return launch_rows_vec<FMT, ROUND, 28>(x, ldx, rows, k, q, ldq, row0, scales, st);
+            if (nv <= 32) return launch_rows_vec<FMT, ROUND, 32>(x, ldx, rows, k, q, ldq, row0, scales, st);
+        }
     }
     hipLaunchKernelGGL((quant_rows_any_kernel<FMT, ROUND, TILED>), dim3((unsigned)rows), dim3(256), 0, st, x, ldx,
                        rows, k, q, ldq, row0, scales);

@@ -331,10 +331,11 @@ def test_int8_rcp_known_answers(ops, device):
     assert s[-1] == 0.0 and not q[-1].any()
 
 
-@pytest.mark.parametrize("rows", [16, 17, 23, 24, 25, 39, 130])
+@pytest.mark.parametrize("rows", [1, 16, 17, 23, 24, 25, 39, 130, 600, 601, 607, 608, 609, 1031])
 @pytest.mark.parametrize("k", [128, 5376])
 def test_tiled_ragged_rows_write_only_their_own(ops, oracle, device, rows, k):
-    """A ragged last unit of the tiled quantizer: its rows' codes and scales
+    """A ragged last unit of the tiled quantizer (from 601 rows on; below, a
+    workgroup per row): its rows' codes and scales
     are the oracle's and nothing past them is written."""
     from _util import from_tiled
 
@@ -351,3 +352,21 @@ def test_tiled_ragged_rows_write_only_their_own(ops, oracle, device, rows, k):
     assert (got[rows:] == 77).all()
     np.testing.assert_array_equal(scales[:rows].cpu().numpy(), rs)
     assert (scales[rows:] == -1.0).all()
+
+
+@pytest.mark.parametrize("fmt,rounding", [("e4m3", "div"), ("int8", "rcp")])
+@pytest.mark.parametrize("rows,k", [(1, 8), (3, 2048), (5, 2056), (601, 6152), (2, 8200), (7, 14344), (3, 16384)])
+def test_rows_of_four_waves(ops, oracle, device, rows, k, fmt, rounding):
+    """A workgroup per row at the edges of its vectors per thread, rows apart, a zero row and one
+    whose maximum is its last element."""
+    print(f"four waves per row {fmt} {rows}x{k}", flush=True)
+    x = activations(rows, k, seed=rows + k)
+    x[-1, -1] = 300.0
+    if rows > 1:
+        x[0] = 0.0
+    wide = torch.full((rows, k + 8), 6.0e4, device=device, dtype=torch.bfloat16)
+    wide[:, :k] = x.to(device)
+    rq, rs = oracle.quant_rows(bits16(x), fmt, rounding)
+    q, s = _run_rows(ops, wide[:, :k], fmt, rounding)
+    np.testing.assert_array_equal(q.view(np.uint8), rq.view(np.uint8))
+    np.testing.assert_array_equal(s, rs)

@@ -69,8 +69,12 @@ int stream_tile(const GemmArgs& a) {
     if (!stream_takes(a)) return 0;
     const StreamChoice best = best_stream_tile(a.m, a.n, a.k);
     if (a.m > kSkinnyMaxM) {
-        // Against the four-wave kernel (or the 16-wave one where K is not a
-        // multiple of 128): 0.78 keeps the calls that gain in both weight
+        // K that is not a multiple of 128 would take the 16-wave kernel, slower in all
+        // of 35 calls of 132 .. 15049 rows, K 272 .. 4064 and N 256 .. 3520: 171 x 272 x
+        // 3824 55 -> 21 us, 11659 x 672 x 3488 205 -> 99, 12403 x 3296 x 1984 200 -> 133,
+        // 13191 x 2080 x 448 58 -> 54 (per-tensor binary16 linears, quantizer included).
+        if (a.k % 128) return best.tile;
+        // Against the four-wave kernel: 0.78 keeps the calls that gain in both weight
         // states (Infinity Cache, HBM) and both layouts; of those left out the
         // best gained 8% in one state and lost 3% in the other.
         return best.cost < 0.78 * four_wave_cost(a) ? best.tile : 0;

@@ -114,3 +114,16 @@ def test_stream_f16_output(ops, oracle, device, m, n, k):
     exact = rsa.astype(np.float64).reshape(-1, 1) * v + bias.double().numpy()  # one rounding each: s_w * acc, the fma
     ref = exact.astype(np.float32).astype(np.float16)
     np.testing.assert_array_equal(out.cpu().numpy().view(np.uint16), ref.view(np.uint16))
+
+
+@pytest.mark.parametrize("m,n,k", [(129, 8, 144), (2600, 1040, 272), (4400, 2056, 656), (130, 4104, 4080)])
+def test_stream_k_tail_at_any_size(ops, oracle, device, m, n, k):
+    """K that is not a multiple of 128 takes this kernel above 128 rows whatever the sizes."""
+    print(f"stream K tail {m}x{n}x{k}", flush=True)
+    x, w, qa, sa, qw, sw = _operands(ops, device, m, n, k, "int8", False, False)
+    out = ops.scaled_mm(qa, qw, sa, sw)
+    torch.cuda.synchronize()
+    rqa, rsa = oracle.quant_rows(bits16(x), "int8", "rcp")
+    rqw, rsw = oracle.quant_rows(bits16(w), "int8", "div")
+    ref = oracle.epilogue(oracle.gemm_i8_i32_fast(rqa, rqw), rsa, rsw, None)
+    np.testing.assert_array_equal(bits16(out), ref)

@@ -696,12 +696,14 @@ namespace {
 
 // Slices of the split (1: no split): with fewer than 128 row blocks of 96 the
 // call has too few workgroups to stream X at HBM speed, so K is cut into
-// slices of at least 4 k-tiles until about 256 workgroups run.
+// slices of at least 4 k-tiles, as many as leave one workgroup per CU: the ring
+// of 140 KiB admits no second, and a 257th starts a second round (3200 rows, 34
+// blocks: 8 slices 22.8 us, 7 slices 16.0; 9000 rows, 3 and 2 slices: 36.2 and 27.0).
 int64_t lora_down_slices(int64_t m, int64_t k, int64_t rank) {
     const int64_t tiles = (m + TileLora96::BM - 1) / TileLora96::BM;
     const int64_t ktiles = (k * 2 + TileLora96::BK - 1) / TileLora96::BK;
     if (tiles >= 128 || rank > TileLora96::BN || rank % 4 || ktiles < 8) return 1;
-    int64_t s = (256 + tiles - 1) / tiles;
+    int64_t s = 256 / tiles;
     if (s > ktiles / 4) s = ktiles / 4;
     const int64_t per = (ktiles + s - 1) / s;
     return (ktiles + per - 1) / per;  // no empty slice

@@ -337,6 +337,12 @@ def test_lora_down_split_over_k(ops, oracle, device, m, k, rank):
     assert rc != 0 and b"workspace" in _lib.lib().h3q_last_error()
 
 
+@pytest.mark.parametrize("m,k,rank", [(8160, 1032, 8), (8161, 1032, 8), (12192, 520, 16)])
+def test_lora_down_slice_counts(ops, oracle, device, m, k, rank):
+    """85 row blocks (three slices), 86 (two) and 127, the last that split."""
+    test_lora_down_split_over_k(ops, oracle, device, m, k, rank)
+
+
 @pytest.mark.parametrize("m,a_tiled", [(512, False), (512, True), (64, False), (16, True)])
 def test_fp8_nan_codes_propagate(ops, device, m, a_tiled):
     """A NaN code (0x7F / 0xFF in e4m3fn) in an activation row makes exactly

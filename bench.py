@@ -885,7 +885,7 @@ def main() -> int:
             "avg_launch_us": round(q_ms * 1e3, 2),
             "in_step_us": round(q_step_ms * 1e3, 2),
             "algorithmic_bytes": q_bytes,
-            "row_major_kernel": "h3q quant_rows_vec_kernel",
+            "row_major_kernel": "h3q quant_rows_wide_kernel",
             "row_major_us": round(q_rm_ms * 1e3, 2),
             "row_major_frac": round(q_bytes / (q_rm_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
         },

@@ -231,7 +231,7 @@ __global__ __launch_bounds__(256) void norm_modulate_quant_kernel(NormQuantArgs 
 #pragma unroll
         for (int i = 0; i < NV; ++i) asm volatile("" : "+v"(v[i].x), "+v"(v[i].y), "+v"(v[i].z), "+v"(v[i].w));
 
-        // Per-token quantization of y, exactly as quant_rows_vec_kernel.
+        // Per-token quantization of y, exactly as the row quantizer.
         const float amax = wave_max(amax_from_packed(m));
         RowQuant<FMT, ROUND> rq;
         rq.init(amax);

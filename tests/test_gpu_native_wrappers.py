@@ -5,10 +5,16 @@ bits (or the same exception) over the argument forms the functions accept."""
 
 from __future__ import annotations
 
+import re
+import shutil
+import subprocess
+import sys
+
 import pytest
 import torch
 
 from _util import activations, weights
+from conftest import ROOT
 
 pytestmark = pytest.mark.gpu
 
@@ -131,3 +137,58 @@ def test_native_wrappers_equal_the_python_ones(ops, device, monkeypatch):
         assert taken == (name not in DECLINED), name
         fa, fb = _flat(a), _flat(b)
         assert len(fa) == len(fb) and all(torch.equal(p, q) for p, q in zip(fa, fb)), name
+
+
+# A kernel library whose h3q_quant_rows returns once another Python thread has
+# run since it was entered (0), or after five seconds without (1).
+_STUB = """
+#include <time.h>
+volatile int entered, released;
+{others}
+int h3q_quant_rows() {{
+    entered = 1;
+    for (int i = 0; i < 5000 && !released; ++i) nanosleep(&(struct timespec){{0, 1000000}}, 0);
+    return !released;
+}}
+"""
+_CHILD = """
+import ctypes, importlib.util, sys, threading, torch
+folder = sys.argv[1]
+stub = ctypes.CDLL(folder + "/libtaomate_h3_amd.so")
+spec = importlib.util.spec_from_file_location("_h3q_torch", folder + "/_h3q_torch.so")
+native = importlib.util.module_from_spec(spec)
+spec.loader.exec_module(native)
+x = torch.zeros(2, 16, device="cuda:0", dtype=torch.bfloat16)
+codes, scales = x.to(torch.int8), torch.zeros(2, 1, device="cuda:0")
+entered, released = (ctypes.c_int.in_dll(stub, name) for name in ("entered", "released"))
+
+def other():
+    while not entered.value:
+        pass
+    released.value = 1
+
+thread = threading.Thread(target=other, daemon=True)
+thread.start()
+result = native.quant_rows(x, 1, 1, codes, scales, 0)
+print("other thread ran" if result is not None else "other thread held up", flush=True)
+released.value = entered.value = 1
+thread.join(10)
+"""
+
+
+def test_native_wrappers_release_the_interpreter_lock(device, tmp_path):
+    """While a wrapper is inside the kernel library another Python thread runs:
+    with a stand-in library (a process of its own, nothing launched) whose entry
+    point waits for one, as a full launch queue waits for the GPU."""
+    from taomate_h3_amd import _lib, _native
+
+    names = set(re.findall(r"\b(h3q_\w+)\s*\(", (ROOT / "include" / "taomate_h3_amd.h").read_text()))
+    others = "\n".join(f"int {name}() {{ return 1; }}" for name in sorted(names - {"h3q_quant_rows"}))
+    (tmp_path / "stub.c").write_text(_STUB.format(others=others))
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(tmp_path / _lib.LIB_PATH.name), str(tmp_path / "stub.c")],
+                   check=True)
+    shutil.copy(_native.PATH, tmp_path)
+    (tmp_path / "child.py").write_text(_CHILD)
+    res = subprocess.run([sys.executable, str(tmp_path / "child.py"), str(tmp_path)], capture_output=True, text=True,
+                         timeout=100)
+    assert res.stdout.strip() == "other thread ran", (res.stdout, res.stderr[-2000:])

@@ -21,7 +21,9 @@
 
 using at::Tensor;
 using Opt = std::optional<Tensor>;
+using OptInt = std::optional<int64_t>;
 using Pair = std::tuple<Tensor, Tensor>;
+using Three = std::tuple<Tensor, Tensor, Tensor>;
 using Triple = std::tuple<Opt, Opt, Opt>;
 
 namespace {
@@ -90,17 +92,15 @@ int scale_kind(const Tensor& s, const Tensor& first, int64_t count) {
     return s.numel() == count ? H3Q_SCALE_PER_ROW : -1;
 }
 
-// m, n: the logical row counts, or -1 for those of a and b.
+// rows_a, rows_b: the logical row counts where they are not those of a and b.
 Opt scaled_mm(const Tensor& a, const Tensor& b, const Tensor& a_scale, const Tensor& b_scale, const Opt& bias,
-              const Opt& lora_t, const Opt& lora_b, double lora_scale, Opt out, bool a_tiled, bool b_tiled, int64_t m,
-              int64_t n, bool f16, int64_t stream) {
+              const Opt& lora_t, const Opt& lora_b, double lora_scale, Opt out, bool a_tiled, bool b_tiled, OptInt rows_a,
+              OptInt rows_b, bool f16, int64_t stream) {
     const at::ScalarType type = a.scalar_type();
     if (!a.is_cuda() || (type != at::kChar && type != at::kFloat8_e4m3fn) || !on(b, a)) return std::nullopt;
     if (!rows_2d(a, type) || !rows_2d(b, type) || b.size(1) != a.size(1)) return std::nullopt;
-    const int64_t k = a.size(1);
-    if (m < 0) m = a.size(0);
-    if (n < 0) n = b.size(0);
-    if (m == 0 || n == 0) return std::nullopt;
+    const int64_t k = a.size(1), m = rows_a.value_or(a.size(0)), n = rows_b.value_or(b.size(0));
+    if (m <= 0 || n <= 0) return std::nullopt;
     const auto held = [](const Tensor& t, int64_t rows, bool tiled) {
         return t.size(0) >= (tiled ? (rows + 15) / 16 * 16 : rows) && (!tiled || t.is_contiguous());
     };
@@ -157,11 +157,12 @@ int64_t table_stride(const Tensor& t, const Tensor& first, int64_t cols) {
     return stride % 8 ? -1 : stride;
 }
 
-// fmt -1: no codes.  Returns (out, codes, scales), None for those not wanted.
+// No fmt: no codes.  Returns (out, codes, scales), None for those not wanted.  gated:
+// (branch, gate, hidden).
 std::optional<Triple> norm_modulate_quant(const Tensor& value, const Tensor& weight, const Tensor& scale,
-                                          const Tensor& shift, const Tensor& indices, double eps, int64_t fmt,
-                                          int64_t rounding, bool want_out, const Opt& branch, const Opt& gate,
-                                          const Opt& hidden, int64_t stream) {
+                                          const Tensor& shift, const Tensor& indices, double eps, OptInt fmt,
+                                          int64_t rounding, bool want_out, const std::optional<Three>& gated,
+                                          int64_t stream) {
     if (!value.is_cuda() || !rows_2d(value, at::kBFloat16) || value.size(0) == 0) return std::nullopt;
     const int64_t rows = value.size(0), cols = value.size(1);
     if (!on(weight, value) || weight.scalar_type() != at::kBFloat16 || weight.numel() != cols || !weight.is_contiguous())
@@ -170,48 +171,49 @@ std::optional<Triple> norm_modulate_quant(const Tensor& value, const Tensor& wei
     if (stride < 0 || table_stride(shift, value, cols) != stride) return std::nullopt;
     if (!on(indices, value) || indices.scalar_type() != at::kLong || indices.numel() != rows || !indices.is_contiguous())
         return std::nullopt;
-    if (fmt >= 0 ? !valid_fmt(fmt) : !want_out) return std::nullopt;
+    if (fmt ? !valid_fmt(*fmt) : !want_out) return std::nullopt;
     const auto matrix = [&](const Tensor& t) {
         return on(t, value) && rows_2d(t, at::kBFloat16) && t.size(0) == rows && t.size(1) == cols;
     };
-    if (branch && !(gate && hidden && matrix(*branch) && matrix(*hidden) && table_stride(*gate, value, cols) == stride))
-        return std::nullopt;
+    const Tensor none;
+    const auto& [branch, gate, hidden] = gated ? *gated : Three(none, none, none);
+    if (gated && !(matrix(branch) && matrix(hidden) && table_stride(gate, value, cols) == stride)) return std::nullopt;
     Opt out, codes, scales;
     if (want_out) out = empty(value, {rows, cols}, at::kBFloat16);
-    if (fmt >= 0) {
-        codes = empty(value, {rows, cols}, code_type(fmt));
+    if (fmt) {
+        codes = empty(value, {rows, cols}, code_type(*fmt));
         scales = empty(value, {rows, 1}, at::kFloat);
     }
     const auto ld = [&](const Tensor& t) { return rows > 1 ? t.stride(0) : cols; };
-    const int f = fmt < 0 ? H3Q_FMT_INT8 : (int)fmt;
+    const int f = (int)fmt.value_or(H3Q_FMT_INT8);
     void* const out_p = out ? out->data_ptr() : nullptr;
     void* const codes_p = codes ? codes->data_ptr() : nullptr;
     float* const scales_p = scales ? floats(*scales) : nullptr;
     const int64_t* const idx = static_cast<const int64_t*>(indices.data_ptr());
     const int rc =
-        branch ? h3q_residual_gate_rms_norm_modulate_quant(
-                     value.data_ptr(), ld(value), branch->data_ptr(), ld(*branch), gate->data_ptr(), weight.data_ptr(),
-                     scale.data_ptr(), shift.data_ptr(), stride, idx, rows, cols, (float)eps, hidden->data_ptr(),
-                     ld(*hidden), out_p, cols, f, (int)rounding, codes_p, cols, scales_p, stream_of(stream))
-               : h3q_rms_norm_modulate_quant(value.data_ptr(), ld(value), weight.data_ptr(), scale.data_ptr(),
-                                             shift.data_ptr(), stride, idx, rows, cols, (float)eps, out_p, cols, f,
-                                             (int)rounding, codes_p, cols, scales_p, stream_of(stream));
+        gated ? h3q_residual_gate_rms_norm_modulate_quant(
+                    value.data_ptr(), ld(value), branch.data_ptr(), ld(branch), gate.data_ptr(), weight.data_ptr(),
+                    scale.data_ptr(), shift.data_ptr(), stride, idx, rows, cols, (float)eps, hidden.data_ptr(),
+                    ld(hidden), out_p, cols, f, (int)rounding, codes_p, cols, scales_p, stream_of(stream))
+              : h3q_rms_norm_modulate_quant(value.data_ptr(), ld(value), weight.data_ptr(), scale.data_ptr(),
+                                            shift.data_ptr(), stride, idx, rows, cols, (float)eps, out_p, cols, f,
+                                            (int)rounding, codes_p, cols, scales_p, stream_of(stream));
     if (rc) return std::nullopt;
     return Triple(out, codes, scales);
 }
 
-std::optional<Triple> swiglu_quant(const Tensor& x, int64_t fmt, int64_t rounding, bool want_out, int64_t stream) {
+std::optional<Triple> swiglu_quant(const Tensor& x, OptInt fmt, int64_t rounding, bool want_out, int64_t stream) {
     if (!x.is_cuda() || !rows_2d(x, at::kBFloat16) || x.size(0) == 0 || x.size(1) % 2) return std::nullopt;
-    if (fmt >= 0 ? !valid_fmt(fmt) : !want_out) return std::nullopt;
+    if (fmt ? !valid_fmt(*fmt) : !want_out) return std::nullopt;
     const int64_t rows = x.size(0), half = x.size(1) / 2;
     Opt out, codes, scales;
     if (want_out) out = empty(x, {rows, half}, at::kBFloat16);
-    if (fmt >= 0) {
-        codes = empty(x, {rows, half}, code_type(fmt));
+    if (fmt) {
+        codes = empty(x, {rows, half}, code_type(*fmt));
         scales = empty(x, {rows, 1}, at::kFloat);
     }
     if (h3q_swiglu_quant(x.data_ptr(), rows > 1 ? x.stride(0) : 2 * half, rows, half, out ? out->data_ptr() : nullptr,
-                         half, fmt < 0 ? H3Q_FMT_INT8 : (int)fmt, (int)rounding, codes ? codes->data_ptr() : nullptr,
+                         half, (int)fmt.value_or(H3Q_FMT_INT8), (int)rounding, codes ? codes->data_ptr() : nullptr,
                          half, scales ? floats(*scales) : nullptr, stream_of(stream)))
         return std::nullopt;
     return Triple(out, codes, scales);

@@ -133,9 +133,8 @@ def norm_modulate_quant(value: torch.Tensor, weight: torch.Tensor, scale: torch.
     quantization (None: no codes).  Returns (out or None, codes or None,
     scales or None)."""
     if codes is None and scales is None and not isinstance(out, torch.Tensor):
-        gated = (None, None, None) if residual_gate is None else residual_gate
-        got = _native_call("norm_modulate_quant", value, weight, scale, shift, indices, eps,
-                           -1 if fmt is None else fmt, rounding, out is True, *gated)
+        got = _native_call("norm_modulate_quant", value, weight, scale, shift, indices, eps, fmt, rounding, out is True,
+                           residual_gate)
         if got is not None:
             return got
     branch = gate = hidden = None
@@ -410,7 +409,7 @@ def swiglu_quant(x: torch.Tensor, *, fmt: int | None = None, rounding: int = ROU
     True to allocate one, None/False for none) and / or per-token codes in
     ``fmt`` (None: no codes).  Returns (out or None, codes or None, scales or None)."""
     if codes is None and scales is None and not isinstance(out, torch.Tensor):
-        got = _native_call("swiglu_quant", x, -1 if fmt is None else fmt, rounding, out is True)
+        got = _native_call("swiglu_quant", x, fmt, rounding, out is True)
         if got is not None:
             return got
     want_out = out is True or isinstance(out, torch.Tensor)
@@ -509,7 +508,7 @@ def scaled_mm(a: torch.Tensor, b: torch.Tensor, a_scale: torch.Tensor, b_scale: 
     they differ from R."""
     if (a_tiled or not is_tiled(a)) and (b_tiled or not is_tiled(b)) and out_dtype in _OUT_F16:
         got = _native_call("scaled_mm", a, b, a_scale, b_scale, bias, lora_t, lora_b, lora_scale, out, a_tiled, b_tiled,
-                           -1 if m is None else m, -1 if n is None else n, _OUT_F16[out_dtype])
+                           m, n, _OUT_F16[out_dtype])
         if got is not None:
             return got
     _require_gpu("scaled_mm", a, b, a_scale, b_scale, bias, lora_t, lora_b, out)

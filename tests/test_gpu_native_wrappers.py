@@ -139,6 +139,34 @@ def test_native_wrappers_equal_the_python_ones(ops, device, monkeypatch):
         assert len(fa) == len(fb) and all(torch.equal(p, q) for p, q in zip(fa, fb)), name
 
 
+def test_native_wrappers_refuse_what_the_python_ones_refuse(ops, device, monkeypatch):
+    """Row counts and formats below zero, and a residual gate without its
+    tensors, are no way to say "not given": the same error as without the
+    native wrapper."""
+    x = activations(37, 512, seed=3).to(device)
+    q, s = ops.quant_rows(x, ops.FMT_INT8)
+    one = torch.ones(1, device=device)
+    table = torch.zeros(1, 512, device=device, dtype=torch.bfloat16)
+    idx = torch.zeros(37, device=device, dtype=torch.int64)
+    g = torch.ones(512, device=device, dtype=torch.bfloat16)
+    norm = lambda **kw: ops.norm_modulate_quant(x, g, table, table, idx, 1e-6, out=True, **kw)  # noqa: E731
+    calls = {
+        "m": lambda: ops.scaled_mm(q, q, one, s, m=-1),
+        "m below": lambda: ops.scaled_mm(q, q, one, s, m=-3),
+        "n": lambda: ops.scaled_mm(q, q, s, one, n=-1),
+        "both scales": lambda: ops.scaled_mm(q, q, s, s, m=-1, n=-1),
+        "norm format": lambda: norm(fmt=-1),
+        "norm gate of nothing": lambda: norm(residual_gate=(None, None, None)),
+        "norm gate without a branch": lambda: norm(residual_gate=(None, table, torch.empty_like(x))),
+        "norm gate without a table": lambda: norm(residual_gate=(x, None, torch.empty_like(x))),
+        "swiglu format": lambda: ops.swiglu_quant(x, fmt=-1, out=True),
+    }
+    for name, call in calls.items():
+        print(name, flush=True)
+        (_, ea), (_, eb), taken = _both(ops, monkeypatch, call)
+        assert eb is not None and ea == eb and not taken, (name, ea, eb)
+
+
 # A kernel library whose h3q_quant_rows returns once another Python thread has
 # run since it was entered (0), or after five seconds without (1).
 _STUB = """

@@ -235,6 +235,23 @@ int h3q_scaled_mm(int format, const void* a, int64_t lda, int a_layout, const fl
                   float lora_scale, void* out, int64_t ldo, int64_t m, int64_t n, int64_t k, void* stream);
 
 /*
+ * The kernels that such a call takes (dense operand rows, a 16-byte aligned out,
+ * lora_rank 0 without an adapter); on the host, for tests and profiles:
+ *   plan[0]     H3Q_GEMM_PER_TILE, _FEW_ROWS (the weight-streaming kernels of m <= 128),
+ *               _STREAM (weight streaming over chip-filling tiles), _FOUR_WAVE, or
+ *               _SPLIT: _FOUR_WAVE for the first columns or rows, then _STREAM
+ *   plan[1..2]  rows and columns of a streaming tile, or 0
+ *   plan[3]     the first columns of a split (negative: its first rows), or 0
+ */
+#define H3Q_GEMM_PER_TILE 0
+#define H3Q_GEMM_FEW_ROWS 1
+#define H3Q_GEMM_STREAM 2
+#define H3Q_GEMM_FOUR_WAVE 3
+#define H3Q_GEMM_SPLIT 4
+int h3q_scaled_mm_plan(int format, int a_layout, int b_layout, int64_t lora_rank, int64_t ldo, int64_t m, int64_t n,
+                       int64_t k, int64_t plan[4]);
+
+/*
  * Raw int32 accumulators of the int8 GEMM: out[m, n] = sum_k a[m, k] * b[n, k]
  * (a [m, k], b [n, k] int8; out int32, ldo elements).  Exposes the integer
  * core of cutlass_scaled_mm (H3/inference/w8a8.py:179-186) for bit-exact

@@ -34,6 +34,7 @@ SIGNATURES: dict[str, tuple[type | None, list]] = {
     "h3q_quant_rows_tiled": (_I, [_P, _I64, _I64, _I64, _I, _I, _I64, _P, _P, _P]),
     "h3q_scaled_mm": (_I, [_I, _P, _I64, _I, _P, _I, _P, _I64, _I, _P, _I, _P, _P, _I64, _P, _I64, _I64, _F, _P,
                            _I64, _I64, _I64, _I64, _P]),
+    "h3q_scaled_mm_plan": (_I, [_I, _I, _I, _I64, _I64, _I64, _I64, _I64, ctypes.POINTER(_I64)]),
     "h3q_gemm_i8_i32": (_I, [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _P]),
     "h3q_lora_down": (_I, [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _P]),
     "h3q_lora_down_workspace_bytes": (_I64, [_I64, _I64, _I64]),

@@ -420,6 +420,34 @@ __attribute__((visibility("default"))) int h3q_scaled_mm(int format, const void*
     return check_launch(h3q::launch_gemm(kind, false, g, (hipStream_t)stream), who);
 }
 
+__attribute__((visibility("default"))) int h3q_scaled_mm_plan(int format, int a_layout, int b_layout, int64_t lora_rank,
+                                                              int64_t ldo, int64_t m, int64_t n, int64_t k,
+                                                              int64_t plan[4]) {
+    const char* who = "h3q_scaled_mm_plan";
+    if (!plan) return fail(H3Q_ERR_INVALID, "%s: null pointer", who);
+    const bool a_tiled = a_layout == H3Q_LAYOUT_TILED, b_tiled = b_layout == H3Q_LAYOUT_TILED;
+    if (m <= 0 || n <= 0) return fail(H3Q_ERR_INVALID, "%s: empty output", who);
+    if (int rc = check_gemm_operands(who, nullptr, k, nullptr, k, m, n, k, 1, a_tiled, b_tiled)) return rc;
+    h3q::GemmArgs g{};
+    g.m = m;
+    g.n = n;
+    g.k = g.lda = g.ldb = k;
+    g.ldo = ldo;
+    g.lora_rank = lora_rank;
+    static const uint16_t some = 0;  // looked at for null only
+    if (lora_rank > 0) g.lora_t = g.lora_b = &some;
+    g.a_tiled = a_tiled;
+    g.b_tiled = b_tiled;
+    g.out_f16 = (format & H3Q_OUT_F16) != 0;
+    const h3q::GemmPlan p = h3q::gemm_plan(g);
+    plan[0] = p.kernel;
+    plan[1] = plan[2] = plan[3] = 0;
+    const int tile = p.kernel == h3q::kGemmSplit ? p.split.tile : p.tile;
+    if (tile) h3q::stream_tile_shape(tile, &plan[1], &plan[2]);
+    if (p.kernel == h3q::kGemmSplit) plan[3] = p.split.columns ? p.split.at : -p.split.at;
+    return ok();
+}
+
 __attribute__((visibility("default"))) int h3q_gemm_i8_i32(const void* a, int64_t lda, const void* b, int64_t ldb,
                                                            void* out, int64_t ldo, int64_t m, int64_t n, int64_t k,
                                                            void* stream) {

@@ -739,17 +739,27 @@ hipError_t launch_lora_down(const GemmArgs& args, void* workspace, int64_t works
     return hipGetLastError();
 }
 
+GemmPlan gemm_plan(const GemmArgs& a) {
+    if (const int tile = stream_tile(a)) return {kGemmStream, tile, {}};
+    if (skinny_supported(a)) return {kGemmFewRows, 0, {}};
+    if (!w4_supported(a)) return {kGemmPerTile, 0, {}};
+    const GemmSplit split = gemm_split(a);
+    return {split.at ? kGemmSplit : kGemmFourWave, 0, split};
+}
+
 hipError_t launch_gemm(int kind, bool raw_i32, const GemmArgs& args, hipStream_t st) {
     GemmArgs a = args;
     a.out_vec = (a.ldo % 4 == 0) && (a.n % 4 == 0) && ((uintptr_t)a.out % 16 == 0);
     const bool lora = a.lora_t != nullptr;
     if (kind != kOpBF16 && !raw_i32) {
-        if (const int tile = stream_tile(a)) return launch_gemm_stream(kind, tile, a, st);
-    }
-    if (kind != kOpBF16 && !raw_i32 && skinny_supported(a)) return launch_gemm_skinny(kind, a, st);
-    if (kind != kOpBF16 && !raw_i32 && w4_supported(a)) {
-        const GemmSplit split = gemm_split(a);
-        return split.at ? launch_gemm_split(kind, split, a, st) : launch_gemm_w4(kind, a, st);
+        const GemmPlan plan = gemm_plan(a);
+        switch (plan.kernel) {
+            case kGemmStream: return launch_gemm_stream(kind, plan.tile, a, st);
+            case kGemmFewRows: return launch_gemm_skinny(kind, a, st);
+            case kGemmFourWave: return launch_gemm_w4(kind, a, st);
+            case kGemmSplit: return launch_gemm_split(kind, plan.split, a, st);
+            case kGemmPerTile: break;
+        }
     }
     if (kind == kOpE4M3)
         return lora ? launch_scaled<TileBigLora, kOpE4M3, true>(a, st) : launch_scaled<TileBig, kOpE4M3, false>(a, st);

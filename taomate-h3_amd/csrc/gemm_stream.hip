@@ -61,10 +61,50 @@ double four_wave_cost(const GemmArgs& a) {
     return 8.0 + a.k / 64.0 * (0.68 * rounds + last);
 }
 
+// Whether the streaming tiles are the faster ones for M <= 128 rows, decided on
+// weights that come from HBM, as a step reads those of each layer (measured on
+// about 900 calls, N 512 .. 16384, K 256 .. 13824, both weight states; below, HBM
+// and in parentheses Infinity Cache, us, gemm_skinny.hip / these tiles).
+//
+// Tiled weights: there a workgroup takes 32 columns and all of A.  Up to 8192
+// columns these are one round, and at 65 .. 128 rows the streaming tiles gain from
+// the cache only (128 x 5120 x 5120 14.3 / 15.3 (12.9 / 10.6), 128 x 2048 x 2048
+// 7.0 / 8.7 (5.5 / 7.2)) until K is long (128 x 5120 x 13824 35.2 / 33.6 (34.8 /
+// 22.6)).  Above, they gain at every K (128 x 10752 x 5376 30.1 / 23.4).  At 33 ..
+// 64 rows a workgroup does half the work and its second round hides more (40 x
+// 10752 x 5376 20.5 / 17.7, 40 x 8208 x 5120 2-6% slower, 40 x 16384 x 4096 3%).
+bool beats_skinny_tiled(int64_t m, int64_t n, int64_t k) {
+    if (m > 64) return n > 8192 || k >= 12288;
+    return m > 32 && n > 10240 && k >= 5120;
+}
+
+// Row-major weights: there a workgroup takes 16 columns and its time grows with
+// the rows; up to 4096 columns each CU gets one, up to 8192 two.  A K that is not a
+// multiple of 128 costs these tiles 10-25%.  32 x 1024 x 3072 6.8 / 9.6, 64 x 2048
+// x 2048 7.5 / 8.5, 64 x 4096 x 5120 18.0 / 17.8 (14.4 / 12.1), 65 x 2048 x 2048 8.6 /
+// 8.4, 65 x 2048 x 3088 10.3 / 11.1, 96 x 2048 x 3088 12.9 / 11.1, 17 x 5120 x 5120
+// 16.6 / 16.1, 17 x 8192 x 5120 17.7 / 18.9, 24 x 5120 x 3072 12.1 / 11.6, 32 x 5120 x
+// 3088 15.3 / 14.4 (9.2 / 10.0), 128 x 5120 x 5120 51 / 18.
+bool beats_skinny_rows(int64_t m, int64_t n, int64_t k) {
+    const bool tail = k % 128 != 0;
+    if (n <= 4096) {
+        if (m > 64) return k >= (!tail ? 2048 : m > 80 ? 3072 : 4096);
+        return m > 56 && k >= 5120;
+    }
+    if (m > 64) return k >= 2048;
+    if (m > 32) return k >= 3072;
+    if (m > 24) return k >= (tail ? 4096 : 3072);
+    if (m <= 16) return false;
+    if (n > 8192) return k >= 3072;
+    return !tail && k >= (n > 6144 ? 7168 : 5120);
+}
+
 }  // namespace
 
-// The rule looks at sizes only (never at the layouts when an adapter is
-// present), so a call gives the same bits whatever layout its operands have.
+// Above 128 rows, and with an adapter at any count, the rule looks at sizes and at
+// the output's alignment, never at the layouts, so there a call gives the same bits
+// whatever layout its operands have.  Up to 128 rows without one the layout of the
+// weights decides, and e4m3 sums may differ in their order between layouts.
 int stream_tile(const GemmArgs& a) {
     if (!stream_takes(a)) return 0;
     const StreamChoice best = best_stream_tile(a.m, a.n, a.k);
@@ -79,19 +119,10 @@ int stream_tile(const GemmArgs& a) {
         // best gained 8% in one state and lost 3% in the other.
         return best.cost < 0.78 * four_wave_cost(a) ? best.tile : 0;
     }
-    // Against the weight-streaming kernels of M <= 128, which take no adapter.
-    if (a.lora_t) return best.tile;  // M = 40, 10752 x 5376, rank 64: 61 us by the per-tile kernel
-    if (a.b_tiled) {
-        // They give every CU 32 columns and all of A: 14.8 against 11.8 us at
-        // 128 x 5120 x 5120, but 10.8 against 11.8 us at M = 64; above 8192
-        // columns their 32-column workgroups no longer fit one round (M = 40,
-        // N = 10752: 20.6 against 14.5 us; N = 5120: 10.2 against 11.3 us).
-        return a.m > 64 || (a.m > 32 && a.n > 8192) ? best.tile : 0;
-    }
-    // Row-major weights: 20 x 5120 x 5120 14.0 against 13.2 us, 100 x 5120 x
-    // 5120 38 against 14 us; short K the other way (64 x 2048 x 2048 7.4 against
-    // 8.1 us, 64 x 1024 x 1040 5.0 against 7.1 us).
-    return (a.m > 16 && a.k >= 3072) || (a.m > 64 && a.k >= 2048) ? best.tile : 0;
+    // M <= 128: against the kernels of gemm_skinny.hip, which take no adapter
+    // (M = 40, 10752 x 5376, rank 64: 61 us by the per-tile kernel).
+    if (a.lora_t || (a.b_tiled ? beats_skinny_tiled(a.m, a.n, a.k) : beats_skinny_rows(a.m, a.n, a.k))) return best.tile;
+    return 0;
 }
 
 // A last round of a few 256 x 256 tiles costs the four-wave kernel 0.51 us per
@@ -153,6 +184,11 @@ hipError_t launch_gemm_split(int kind, const GemmSplit& split, const GemmArgs& a
     }
     const hipError_t e = launch_gemm_w4(kind, head, st);
     return e != hipSuccess ? e : launch_gemm_stream(kind, split.tile, rest, st);
+}
+
+void stream_tile_shape(int tile, int64_t* rows, int64_t* columns) {
+    for (const StreamTile& t : kTiles)
+        if (t.id == tile) *rows = t.bm, *columns = t.bn;
 }
 
 hipError_t launch_gemm_stream(int kind, int tile, const GemmArgs& a, hipStream_t st) {

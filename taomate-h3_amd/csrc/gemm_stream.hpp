@@ -42,9 +42,10 @@
 //   592 x 10752 x 5376     48.9 / 50.3    32.8 / 37.9
 //   1043 x 5120 x 5120     46.6 / 47.0    27.0 / 33.5
 //   1376 x 5120 x 13824    112  / 114     88.2 / 91.4
-// and against the weight-streaming kernel of M <= 128 (gemm_skinny.hip):
-//   100 x 10752 x 5376     29.6 / 30.0    16.3 / 23.4
-//   128 x 5120 x 5120      14.8 / 14.9    11.8 / 15.2
+// and against the weight-streaming kernel of M <= 128 (gemm_skinny.hip), which keeps
+// the second of these (gemm_stream.hip):
+//   112 x 10752 x 5376     28.9 / 29.4    15.9 / 22.9
+//   128 x 5120 x 5120      12.9 / 14.3    10.6 / 15.3
 #pragma once
 
 #include <stdint.h>

@@ -114,6 +114,7 @@ hipError_t launch_gemm_skinny(int kind, const GemmArgs& a, hipStream_t st);
 // multiples of 8, a 16-byte aligned output.  stream_tile gives the tile to use
 // (0: another kernel is the better one); launch_gemm routes there itself.
 int stream_tile(const GemmArgs& a);
+void stream_tile_shape(int tile, int64_t* rows, int64_t* columns);
 hipError_t launch_gemm_stream(int kind, int tile, const GemmArgs& a, hipStream_t st);
 
 // A call in two launches: its first columns (or rows) in full rounds of the
@@ -126,6 +127,16 @@ struct GemmSplit {
 };
 GemmSplit gemm_split(const GemmArgs& a);
 hipError_t launch_gemm_split(int kind, const GemmSplit& split, const GemmArgs& a, hipStream_t st);
+
+// The kernels of a scaled e4m3 / int8 call (values of include/taomate_h3_amd.h):
+// launch_gemm follows it.
+enum GemmKernel : int { kGemmPerTile = 0, kGemmFewRows = 1, kGemmStream = 2, kGemmFourWave = 3, kGemmSplit = 4 };
+struct GemmPlan {
+    GemmKernel kernel;
+    int tile;         // kGemmStream
+    GemmSplit split;  // kGemmSplit
+};
+GemmPlan gemm_plan(const GemmArgs& a);
 
 // Fused RMSNorm + AdaLN modulate (+ residual gate) + per-token quantization
 // (norm_quant.hip).  All bf16 tensors are row-major with element strides;

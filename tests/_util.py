@@ -2,8 +2,23 @@
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import torch
+
+GEMM_KERNELS = ("per tile", "few rows", "stream", "four waves", "split")
+
+
+def gemm_plan(m: int, n: int, k: int, *, a_tiled: bool = False, b_tiled: bool = False, rank: int = 0,
+              f16: bool = False, ldo: int | None = None):
+    """(kernel, streaming tile (rows, columns), split) of a scaled GEMM call, as the library routes it."""
+    from taomate_h3_amd import _lib
+
+    plan = (ctypes.c_int64 * 4)()
+    _lib.call("h3q_scaled_mm_plan", 0x100 if f16 else 0, int(a_tiled), int(b_tiled), rank, n if ldo is None else ldo,
+              m, n, k, plan)
+    return GEMM_KERNELS[plan[0]], (plan[1], plan[2]), plan[3]
 
 
 def bits16(t: torch.Tensor) -> np.ndarray:

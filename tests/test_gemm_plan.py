@@ -1,0 +1,44 @@
+"""Which kernels a scaled GEMM call takes (h3q_scaled_mm_plan, on the host): the
+sizes on both sides of every line of the rules, so that a change of a rule shows
+here and not only in a measurement."""
+
+from __future__ import annotations
+
+import pytest
+
+from _util import gemm_plan
+
+FEW, STREAM = "few rows", "stream"
+
+
+@pytest.mark.parametrize("m,n,k,kernel", [
+    # 65 .. 128 rows: up to 8192 columns the few-rows kernel until K is long
+    (128, 5120, 5120, FEW), (65, 5120, 5120, FEW), (128, 2048, 2048, FEW), (96, 8192, 10240, FEW),
+    (128, 5120, 12288, STREAM), (128, 5120, 13824, STREAM), (65, 8200, 256, STREAM), (77, 10752, 5376, STREAM),
+    # 33 .. 64 rows: streaming tiles for wide weights with K from 5120
+    (40, 10752, 5376, STREAM), (64, 10248, 5120, STREAM), (64, 10240, 5120, FEW), (40, 16384, 4096, FEW),
+    (40, 8208, 5120, FEW), (64, 5120, 13824, FEW),
+    (32, 16384, 13824, FEW), (1, 10752, 5376, FEW)])
+def test_few_rows_tiled_weights(m, n, k, kernel):
+    assert gemm_plan(m, n, k, a_tiled=True, b_tiled=True)[0] == kernel
+    assert gemm_plan(m, n, k, b_tiled=True)[0] == kernel
+
+
+@pytest.mark.parametrize("m,n,k,kernel", [
+    (16, 10752, 13824, FEW), (17, 10752, 3072, STREAM), (17, 10752, 2944, FEW),
+    (17, 5120, 5120, STREAM), (17, 5120, 4992, FEW), (24, 8192, 5120, FEW), (24, 8192, 7168, STREAM),
+    (24, 5120, 13840, FEW), (25, 5120, 3072, STREAM), (32, 5120, 3088, FEW), (32, 5120, 4112, STREAM),
+    (32, 4096, 13824, FEW), (48, 1024, 3072, FEW), (56, 4096, 13824, FEW), (57, 4096, 5120, STREAM),
+    (33, 4104, 3072, STREAM), (33, 4104, 2944, FEW),
+    (65, 1024, 2048, STREAM), (65, 1024, 1920, FEW), (65, 1024, 2064, FEW), (65, 2048, 3088, FEW),
+    (65, 2048, 4112, STREAM), (81, 2048, 3088, STREAM), (128, 2048, 2064, FEW), (65, 5120, 2064, STREAM),
+    (128, 5120, 1920, FEW)])
+def test_few_rows_row_major_weights(m, n, k, kernel):
+    assert gemm_plan(m, n, k)[0] == kernel
+
+
+def test_few_rows_with_an_adapter():
+    """The few-rows kernels take no adapter: streaming tiles where their form allows, else per tile."""
+    assert gemm_plan(16, 5120, 5120, b_tiled=True, rank=64)[0] == STREAM
+    assert gemm_plan(128, 2048, 2048, rank=8)[0] == STREAM
+    assert gemm_plan(16, 5116, 5120, b_tiled=True, rank=64)[0] == "per tile"

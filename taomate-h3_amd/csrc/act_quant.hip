@@ -32,8 +32,8 @@ __device__ __forceinline__ int64_t code_offset(int64_t row, int64_t k, int64_t l
 }
 
 // Vector path: K % 8 == 0, x rows 16-byte aligned, q rows 8-byte aligned, K <= NV*512.
-// Codes go to the tiled layout at absolute row row0 + row, a wave per row.
-template <int FMT, int ROUND, int NV>
+// A wave per row; TILED: codes go to the tiled layout at absolute row row0 + row.
+template <int FMT, int ROUND, int NV, bool TILED>
 __global__ __launch_bounds__(256) void quant_rows_vec_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                              int64_t rows, int k, uint8_t* __restrict__ q,
                                                              int64_t ldq, int64_t row0,
@@ -70,17 +70,17 @@ __global__ __launch_bounds__(256) void quant_rows_vec_kernel(const uint16_t* __r
                 uint2 out;
                 out.x = rq.pack4(v[i].x, v[i].y);
                 out.y = rq.pack4(v[i].z, v[i].w);
-                *reinterpret_cast<uint2*>(q + code_offset<true>(row0 + row, 8 * (int64_t)vec, ldq)) = out;
+                *reinterpret_cast<uint2*>(q + code_offset<TILED>(row0 + row, 8 * (int64_t)vec, ldq)) = out;
             }
         }
         if (lane == 0) scales[row] = rq.s;
     }
 }
 
-// Row-major codes, and tiled codes of few rows: a workgroup of four waves per
-// row, NV vectors per thread (K <= NV * 2048), so that a quarter of the row's loads
-// and conversions stands in each wave's chain and rows in flight fill the chip at
-// a quarter of the registers.  Same alignment; TILED as above.
+// Row-major codes of long rows, and tiled codes of few rows: a workgroup of four
+// waves per row, NV vectors per thread (K <= NV * 2048), so that a quarter of the
+// row's loads and conversions stands in each wave's chain and rows in flight fill the
+// chip at a quarter of the registers.  Same alignment; TILED as above.
 template <int FMT, int ROUND, int NV, bool TILED>
 __global__ __launch_bounds__(256) void quant_rows_wide_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                               int64_t rows, int k, uint8_t* __restrict__ q,
@@ -261,16 +261,29 @@ constexpr int64_t kWideBlocks = 1 << 20;
 // whose one unit per CU serializes load, conversion and store: 16 x 5120 4.9 against
 // 2.9 us, 77 x 5376 6.1 / 3.1, 200 x 7168 6.4 / 3.9, 400 x 14336 12.0 / 7.8; even at 800 rows
 // (K = 5120 6.2 / 6.2, 7168 7.9 / 7.5, 14336 13.3 / 13.8), where its 8-byte stores into
-// 16-row blocks begin to cost (1600 x 5120 8.2 / 9.6).
-constexpr int64_t kWideTiledRows = 600;
+// 16-row blocks begin to cost (1600 x 5120 8.2 / 9.6).  Shorter rows have less to share
+// (257 x 2048 3.4 / 3.1, 400 x 3584 4.4 / 4.2, 512 x 2048 3.5 / 3.7, 592 x 3584 5.1 / 5.2), and
+// up to K = 1024 two or three of the four waves nothing (1 x 512 2.1 / 2.0, 16 x 512 2.2 /
+// 2.3, 592 x 1024 2.9 / 3.3).
+static int64_t wide_tiled_rows(int64_t k) { return k <= 1024 ? 8 : (k <= 3584 ? 384 : 600); }
 
-template <int FMT, int ROUND, int NV>
+// Row-major codes that a wave per row writes faster than a workgroup per row: rows
+// too short for four waves (24576 x 512 10.6 against 20.7 us, 3200 x 1024 4.6 / 5.7),
+// and many rows of a few vectors per lane, where the wave's own loads fill the chip
+// (8192 x 2048 10.4 / 12.2, 3200 x 2048 6.6 / 6.9, 1043 x 2048 4.1 / 3.9; 8192 x 3072 14.4 /
+// 15.4, 3200 x 3072 8.6 / 8.2).  Longer rows stay with the workgroup: 16 x 5120 3.6 / 2.8
+// us, 400 x 14336 8.4 / 5.2, 3200 x 5120 11.7 / 9.5, 24576 x 14336 202 / 192.
+static bool wave_per_row(int64_t rows, int64_t k) {
+    return k <= 1024 || (k <= 2048 && rows > 2048) || (k <= 3072 && rows > 4096);
+}
+
+template <int FMT, int ROUND, int NV, bool TILED>
 static hipError_t launch_rows_vec(const uint16_t* x, int64_t ldx, int64_t rows, int64_t k, uint8_t* q,
                                   int64_t ldq, int64_t row0, float* scales, hipStream_t st) {
     // One wave per row up to 4 waves per SIMD of the chip (1024 workgroups of
     // four waves on 256 CUs); beyond that each wave takes several rows.
     const int64_t blocks = (rows + 3) / 4 < kRowBlocks ? (rows + 3) / 4 : kRowBlocks;
-    hipLaunchKernelGGL((quant_rows_vec_kernel<FMT, ROUND, NV>), dim3((unsigned)blocks), dim3(256), 0, st, x,
+    hipLaunchKernelGGL((quant_rows_vec_kernel<FMT, ROUND, NV, TILED>), dim3((unsigned)blocks), dim3(256), 0, st, x,
                        ldx, rows, (int)k, q, ldq, row0, scales);
     return hipGetLastError();
 }
@@ -333,10 +346,15 @@ static hipError_t dispatch_rows(const uint16_t* x, int64_t ldx, int64_t rows, in
     const bool aligned = (k % 8 == 0) && (ldx % 8 == 0) && (TILED || ldq % 8 == 0) &&
                          ((uintptr_t)x % 16 == 0) && ((uintptr_t)q % 8 == 0);
     const int64_t nv = (k + 511) / 512;
-    // Row-major: always the workgroup per row; a wave per row measured 3.6 against 2.8
-    // us at 16 x 5120, 8.4 / 5.2 at 400 x 14336, 11.7 / 9.5 at 3200 x 5120, 202 / 192 at
-    // 24576 x 14336.
-    if (aligned && nv <= 32 && (!TILED || rows <= kWideTiledRows)) {
+    if constexpr (!TILED) {
+        if (aligned && wave_per_row(rows, k)) {
+            if (nv <= 1) return launch_rows_vec<FMT, ROUND, 1, false>(x, ldx, rows, k, q, ldq, row0, scales, st);
+            if (nv <= 2) return launch_rows_vec<FMT, ROUND, 2, false>(x, ldx, rows, k, q, ldq, row0, scales, st);
+            if (nv <= 4) return launch_rows_vec<FMT, ROUND, 4, false>(x, ldx, rows, k, q, ldq, row0, scales, st);
+            return launch_rows_vec<FMT, ROUND, 6, false>(x, ldx, rows, k, q, ldq, row0, scales, st);
+        }
+    }
+    if (aligned && nv <= 32 && (!TILED || rows <= wide_tiled_rows(k))) {
         if (nv <= 4) return launch_rows_wide<FMT, ROUND, 1, TILED>(x, ldx, rows, k, q, ldq, row0, scales, st);
         if (nv <= 8) return launch_rows_wide<FMT, ROUND, 2, TILED>(x, ldx, rows, k, q, ldq, row0, scales, st);
         if (nv <= 12) return launch_rows_wide<FMT, ROUND, 3, TILED>(x, ldx, rows, k, q, ldq, row0, scales, st);
@@ -352,16 +370,16 @@ static hipError_t dispatch_rows(const uint16_t* x, int64_t ldx, int64_t rows, in
         if (aligned && nv <= 32 && row0 % 16 == 0 && (uintptr_t)q % 16 == 0)
             return dispatch_rows_tiled_img<FMT, ROUND>(x, ldx, rows, k, q, row0, scales, st);
         if (aligned) {
-            if (nv <= 2) return launch_rows_vec<FMT, ROUND, 2>(x, ldx, rows, k, q, ldq, row0, scales, st);
-            if (nv <= 4) return launch_rows_vec<FMT, ROUND, 4>(x, ldx, rows, k, q, ldq, row0, scales, st);
-            if (nv <= 8) return launch_rows_vec<FMT, ROUND, 8>(x, ldx, rows, k, q, ldq, row0, scales, st);
-            if (nv <= 10) return launch_rows_vec<FMT, ROUND, 10>(x, ldx, rows, k, q, ldq, row0, scales, st);
-            if (nv <= 11) return launch_rows_vec<FMT, ROUND, 11>(x, ldx, rows, k, q, ldq, row0, scales, st);
-            if (nv <= 14) return launch_rows_vec<FMT, ROUND, 14>(x, ldx, rows, k, q, ldq, row0, scales, st);
-            if (nv <= 16) return launch_rows_vec<FMT, ROUND, 16>(x, ldx, rows, k, q, ldq, row0, scales, st);
-            if (nv <= 24) return launch_rows_vec<FMT, ROUND, 24>(x, ldx, rows, k, q, ldq, row0, scales, st);
-            if (nv <= 28) return launch_rows_vec<FMT, ROUND, 28>(x, ldx, rows, k, q, ldq, row0, scales, st);
-            if (nv <= 32) return launch_rows_vec<FMT, ROUND, 32>(x, ldx, rows, k, q, ldq, row0, scales, st);
+            if (nv <= 2) return launch_rows_vec<FMT, ROUND, 2, true>(x, ldx, rows, k, q, ldq, row0, scales, st);
+            if (nv <= 4) return launch_rows_vec<FMT, ROUND, 4, true>(x, ldx, rows, k, q, ldq, row0, scales, st);
+            if (nv <= 8) return launch_rows_vec<FMT, ROUND, 8, true>(x, ldx, rows, k, q, ldq, row0, scales, st);
+            if (nv <= 10) return launch_rows_vec<FMT, ROUND, 10, true>(x, ldx, rows, k, q, ldq, row0, scales, st);
+            if (nv <= 11) return launch_rows_vec<FMT, ROUND, 11, true>(x, ldx, rows, k, q, ldq, row0, scales, st);
+            if (nv <= 14) return launch_rows_vec<FMT, ROUND, 14, true>(x, ldx, rows, k, q, ldq, row0, scales, st);
+            if (nv <= 16) return launch_rows_vec<FMT, ROUND, 16, true>(x, ldx, rows, k, q, ldq, row0, scales, st);
+            if (nv <= 24) return launch_rows_vec<FMT, ROUND, 24, true>(x, ldx, rows, k, q, ldq, row0, scales, st);
+            if (nv <= 28) return launch_rows_vec<FMT, ROUND, 28, true>(x, ldx, rows, k, q, ldq, row0, scales, st);
+            if (nv <= 32) return launch_rows_vec<FMT, ROUND, 32, true>(x, ldx, rows, k, q, ldq, row0, scales, st);
         }
     }
     hipLaunchKernelGGL((quant_rows_any_kernel<FMT, ROUND, TILED>), dim3((unsigned)rows), dim3(256), 0, st, x, ldx,

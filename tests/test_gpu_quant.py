@@ -334,9 +334,9 @@ def test_int8_rcp_known_answers(ops, device):
 @pytest.mark.parametrize("rows", [1, 16, 17, 23, 24, 25, 39, 130, 600, 601, 607, 608, 609, 1031])
 @pytest.mark.parametrize("k", [128, 5376])
 def test_tiled_ragged_rows_write_only_their_own(ops, oracle, device, rows, k):
-    """A ragged last unit of the tiled quantizer (from 601 rows on; below, a
-    workgroup per row): its rows' codes and scales
-    are the oracle's and nothing past them is written."""
+    """A ragged last unit of the tiled quantizer (K = 128; K = 5376 from 601 rows
+    on, below it a workgroup per row): its rows' codes and scales are the oracle's
+    and nothing past them is written."""
     from _util import from_tiled
 
     print(f"tiled ragged {rows}x{k}", flush=True)
@@ -370,3 +370,18 @@ def test_rows_of_four_waves(ops, oracle, device, rows, k, fmt, rounding):
     q, s = _run_rows(ops, wide[:, :k], fmt, rounding)
     np.testing.assert_array_equal(q.view(np.uint8), rq.view(np.uint8))
     np.testing.assert_array_equal(s, rs)
+
+
+@pytest.mark.parametrize("fmt,rounding", [("e4m3", "div"), ("int8", "rcp")])
+@pytest.mark.parametrize("rows,k", [(1, 512), (4103, 520), (6, 1024), (2048, 1032), (2049, 2048), (4096, 2056),
+                                    (4097, 3072), (4101, 3080)])
+def test_rows_of_one_wave(ops, oracle, device, rows, k, fmt, rounding):
+    """Both sides of the row counts and widths from which a wave takes a row of its own."""
+    test_rows_of_four_waves(ops, oracle, device, rows, k, fmt, rounding)
+
+
+@pytest.mark.parametrize("rows", [1, 8, 9, 384, 385, 399])
+@pytest.mark.parametrize("k", [1024, 1152, 3584, 3712])
+def test_tiled_codes_of_short_rows(ops, oracle, device, rows, k):
+    """Both sides of the widths and row counts between the tiled kernels, nothing past the rows written."""
+    test_tiled_ragged_rows_write_only_their_own(ops, oracle, device, rows, k)

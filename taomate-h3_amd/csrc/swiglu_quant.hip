@@ -23,11 +23,12 @@
 // where its own exp (the library's, or Triton's) moves the binary32 silu
 // across a bf16 rounding boundary.
 //
-// Several waves share a row, y kept in VGPRs (8-element vectors) for the
-// quantizer, so that even a few rows spread over the chip.
+// A row is shared by as many waves as it fills, y kept in VGPRs (8-element vectors)
+// for the quantizer, so that even a few long rows spread over the chip.
 // Per row 4F bytes in, F bytes of codes + 4 bytes of scale out (+ 2F with out).
 //
-// Table form (swiglu_quant_lut_kernel, calls of at least kLutMinRows rows).
+// Table form (swiglu_quant_lut_kernel, from a row count that depends on the row's
+// length, see launch_sq_fmt).
 // Because s is a function of the 16-bit gate pattern alone, the library
 // evaluates it once per device for all 65536 patterns (silu_table_kernel,
 // the same instructions as above) into a 128 KiB table in device memory.
@@ -78,16 +79,22 @@ __global__ __launch_bounds__(256) void silu_table_kernel(uint16_t* __restrict__ 
     reinterpret_cast<uint32_t*>(table)[g >> 1] = pack_bf16x2(silu_f32(bf16_lo(w)), silu_f32(bf16_hi(w)));
 }
 
-// Direct form: a workgroup of four waves per row, NV vectors per lane each: wave w
-// takes vectors (4 i + w) * 64 + lane, and the row's maximum is exchanged through
-// LDS (double-buffered by row parity, so one barrier a row).
-template <int FMT, int ROUND, int NV>
+// Direct form: workgroups of four waves, SPLIT waves to a row, NV vectors per lane
+// each: wave `part` of a row takes vectors (SPLIT i + part) * 64 + lane, and the row's
+// maximum is exchanged through LDS (double-buffered by parity, so one barrier a
+// group of rows; a wave of its own needs none).
+template <int FMT, int ROUND, int NV, int SPLIT>
 __global__ __launch_bounds__(256) void swiglu_quant_kernel(SwigluQuantArgs p) {
     __shared__ uint32_t red[2][4];
+    constexpr int kRows = 4 / SPLIT;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int part = wave % SPLIT, sub = wave / SPLIT;
     const int nvec = p.half >> 3;
     int parity = 0;
-    for (int64_t row = blockIdx.x; row < p.rows; row += gridDim.x) {
+    const int64_t groups = (p.rows + kRows - 1) / kRows;
+    for (int64_t group = blockIdx.x; group < groups; group += gridDim.x) {
+        const int64_t row = group * kRows + sub;
+        const bool live = row < p.rows;
         const uint4* gr = reinterpret_cast<const uint4*>(p.x + row * p.ldx);
         const uint4* ur = reinterpret_cast<const uint4*>(p.x + row * p.ldx + p.half);
         uint4 y[NV];
@@ -98,8 +105,8 @@ __global__ __launch_bounds__(256) void swiglu_quant_kernel(SwigluQuantArgs p) {
             uint4 g[B], u[B];
 #pragma unroll
             for (int b = 0; b < B; ++b) {
-                const int vec = ((i0 + b) * 4 + wave) * 64 + lane;
-                const bool in = i0 + b < NV && vec < nvec;
+                const int vec = ((i0 + b) * SPLIT + part) * 64 + lane;
+                const bool in = live && i0 + b < NV && vec < nvec;
                 g[b] = in ? gr[vec] : make_uint4(0, 0, 0, 0);
                 u[b] = in ? ur[vec] : make_uint4(0, 0, 0, 0);
             }
@@ -118,27 +125,30 @@ __global__ __launch_bounds__(256) void swiglu_quant_kernel(SwigluQuantArgs p) {
                 m = pk_abs_max(m, y[i0 + b].w);
             }
         }
-        if (p.out) {
+        if (p.out && live) {
             uint4* orow = reinterpret_cast<uint4*>(p.out + row * p.ldo);
 #pragma unroll
             for (int i = 0; i < NV; ++i) {
-                const int vec = (4 * i + wave) * 64 + lane;
+                const int vec = (SPLIT * i + part) * 64 + lane;
                 if (vec < nvec) orow[vec] = y[i];
             }
         }
         if (p.codes == nullptr) continue;
-        const float mine = wave_max(amax_from_packed(m));
-        if (lane == 0) red[parity][wave] = __float_as_uint(mine);
-        __syncthreads();
-        float amax = 0.0f;
+        float amax = wave_max(amax_from_packed(m));
+        if constexpr (SPLIT > 1) {
+            if (lane == 0) red[parity][wave] = __float_as_uint(amax);
+            __syncthreads();
+            amax = 0.0f;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) amax = mag_max(amax, __uint_as_float(red[parity][w]));
-        parity ^= 1;
+            for (int w = 0; w < SPLIT; ++w) amax = mag_max(amax, __uint_as_float(red[parity][sub * SPLIT + w]));
+            parity ^= 1;
+        }
+        if (!live) continue;
         RowQuant<FMT, ROUND> rq;
         rq.init(amax);
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
-            const int vec = (4 * i + wave) * 64 + lane;
+            const int vec = (SPLIT * i + part) * 64 + lane;
             if (vec < nvec) {
                 uint2 o;
                 o.x = rq.pack4(y[i].x, y[i].y);
@@ -146,7 +156,7 @@ __global__ __launch_bounds__(256) void swiglu_quant_kernel(SwigluQuantArgs p) {
                 *reinterpret_cast<uint2*>(p.codes + row * p.ldq + 8 * (int64_t)vec) = o;
             }
         }
-        if (threadIdx.x == 0) p.scales[row] = rq.s;
+        if (lane == 0 && part == 0) p.scales[row] = rq.s;
     }
 }
 
@@ -154,8 +164,8 @@ __global__ __launch_bounds__(256) void swiglu_quant_kernel(SwigluQuantArgs p) {
 // the LDS), SPLIT waves to a row, so a workgroup takes groups of 16 / SPLIT rows
 // blockIdx.x, blockIdx.x + grid, ...  The next group's gate and up are requested
 // before the barrier that exchanges this group's maxima, so reads and stores
-// overlap.  Measured on MI355X (int8 codes, inputs rotated, us; a wave per row as
-// before -> this): 2640 x 7168 26.4 -> 22.3, 8192 x 7168 59.6 -> 53.9, 8192 x 13824
+// overlap.  Measured on MI355X (int8 codes, inputs rotated, us; a wave per row of any
+// length -> this): 2640 x 7168 26.4 -> 22.3, 8192 x 7168 59.6 -> 53.9, 8192 x 13824
 // 119.4 -> 108.4 (5.2 TB/s, the rate of a large copy), 4000 x 14336 58.9 -> 54.5.
 constexpr int kLutWaves = 16;
 template <int FMT, int ROUND, int NV, int SPLIT>
@@ -217,14 +227,16 @@ __global__ __launch_bounds__(kLutWaves * 64) void swiglu_quant_lut_kernel(Swiglu
             m = pk_abs_max(m, y[i].w);
         }
         load(group + gridDim.x);
-        const float mine = wave_max(amax_from_packed(m));
-        if (lane == 0) red[parity][wave] = __float_as_uint(mine);
-        // (not __syncthreads: the next group's loads stay in flight)
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        float amax = 0.0f;
+        float amax = wave_max(amax_from_packed(m));
+        if constexpr (SPLIT > 1) {
+            if (lane == 0) red[parity][wave] = __float_as_uint(amax);
+            // (not __syncthreads: the next group's loads stay in flight)
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            amax = 0.0f;
 #pragma unroll
-        for (int w = 0; w < SPLIT; ++w) amax = mag_max(amax, __uint_as_float(red[parity][sub * SPLIT + w]));
-        parity ^= 1;
+            for (int w = 0; w < SPLIT; ++w) amax = mag_max(amax, __uint_as_float(red[parity][sub * SPLIT + w]));
+            parity ^= 1;
+        }
         if (row >= p.rows) continue;
         if (p.out) {
             uint4* orow = reinterpret_cast<uint4*>(p.out + row * p.ldo);
@@ -252,12 +264,6 @@ __global__ __launch_bounds__(kLutWaves * 64) void swiglu_quant_lut_kernel(Swiglu
 }
 
 namespace {
-
-// Calls of at least this many rows take the table form; below it the table's copy
-// into every workgroup's LDS is not paid back (F = 7168: 128 rows 5.5 us by the
-// table, 4.7 us direct, 300 rows 6.2 / 7.1 us; F = 14336: 7.7 / 6.8 and 9.0 / 10.8 us).
-// A wave per row, the form before, took 10.1 and 11.0 us, 17.3 and 18.0 us.
-constexpr int64_t kLutMinRows = 192;
 
 // The current device's table, filled on first use (launch + wait, once per
 // device), and its CU count; null while a graph is being captured on st and
@@ -303,39 +309,51 @@ hipError_t silu_table_for(hipStream_t st, const uint16_t** out, int* cus) {
     return hipSuccess;
 }
 
-// ND: vectors per lane of the direct form (four waves a row); NT, SPLIT: those of
-// the table form.
-template <int FMT, int ROUND, int ND, int NT, int SPLIT>
-hipError_t launch_sq_nv(const SwigluQuantArgs& a, hipStream_t st) {
-    if (a.rows >= kLutMinRows) {
+// ND, SD: vectors per lane and waves per row of the direct form; NT, ST: those of the
+// table form, which takes calls of at least `table_rows` rows.
+template <int FMT, int ROUND, int ND, int SD, int NT, int ST>
+hipError_t launch_sq_nv(const SwigluQuantArgs& a, int64_t table_rows, hipStream_t st) {
+    if (a.rows >= table_rows) {
         const uint16_t* table = nullptr;
         int cus = 0;
         const hipError_t e = silu_table_for(st, &table, &cus);
         if (e != hipSuccess) return e;
         if (table) {
-            constexpr int kRows = kLutWaves / SPLIT;
+            constexpr int kRows = kLutWaves / ST;
             const int64_t groups = (a.rows + kRows - 1) / kRows;
             const int64_t blocks = groups < cus ? groups : cus;
-            hipLaunchKernelGGL((swiglu_quant_lut_kernel<FMT, ROUND, NT, SPLIT>), dim3((unsigned)blocks),
+            hipLaunchKernelGGL((swiglu_quant_lut_kernel<FMT, ROUND, NT, ST>), dim3((unsigned)blocks),
                                dim3(kLutWaves * 64), 0, st, a, table);
             return hipGetLastError();
         }
     }
     constexpr int64_t kBlocks = 8192;
-    const int64_t blocks = a.rows < kBlocks ? a.rows : kBlocks;
-    hipLaunchKernelGGL((swiglu_quant_kernel<FMT, ROUND, ND>), dim3((unsigned)blocks), dim3(256), 0, st, a);
+    constexpr int kRows = 4 / SD;
+    const int64_t groups = (a.rows + kRows - 1) / kRows;
+    const int64_t blocks = groups < kBlocks ? groups : kBlocks;
+    hipLaunchKernelGGL((swiglu_quant_kernel<FMT, ROUND, ND, SD>), dim3((unsigned)blocks), dim3(256), 0, st, a);
     return hipGetLastError();
 }
 
+// By the row's length: as many waves to a row as it fills, and the row count from
+// which the table is paid back.  Its copy into every workgroup's LDS takes 2-3 us, so
+// short rows, whose direct form runs at the same rate, need many (us, direct / table):
+// F = 512 2640 rows 4.9 / 5.8, 8192 8.0 / 8.0, 20000 14.2 / 13.2; F = 1024 2640 6.7 / 7.5,
+// 8192 12.3 / 11.4; F = 2048 2640 9.4 / 10.3, 8192 21.9 / 19.2; F = 3584 800 7.5 / 7.6, 1043 8.5 /
+// 9.6 (a second round of 1024 rows), 2640 14.1 / 13.4; F = 7168 128 4.7 / 5.5, 300 7.1 / 6.2;
+// F = 14336 6.8 / 7.7 and 10.8 / 9.0.  Four waves to every row took 15.7 us at 8192 x 512
+// directly and 16.4 by the table, 17.0 and 17.5 at 8192 x 1024.
 template <int FMT, int ROUND>
 hipError_t launch_sq_fmt(const SwigluQuantArgs& a, hipStream_t st) {
     const int nvec = a.half / 8;
-    if (nvec <= 256) return launch_sq_nv<FMT, ROUND, 1, 1, 4>(a, st);
-    if (nvec <= 512) return launch_sq_nv<FMT, ROUND, 2, 2, 4>(a, st);
-    if (nvec <= 1024) return launch_sq_nv<FMT, ROUND, 4, 2, 8>(a, st);
-    if (nvec <= 1536) return launch_sq_nv<FMT, ROUND, 6, 3, 8>(a, st);
-    if (nvec <= 1792) return launch_sq_nv<FMT, ROUND, 7, 4, 8>(a, st);
-    return launch_sq_nv<FMT, ROUND, 8, 4, 8>(a, st);
+    if (nvec <= 64) return launch_sq_nv<FMT, ROUND, 1, 1, 1, 1>(a, 8192, st);
+    if (nvec <= 128) return launch_sq_nv<FMT, ROUND, 1, 2, 2, 1>(a, 5120, st);
+    if (nvec <= 256) return launch_sq_nv<FMT, ROUND, 1, 4, 2, 2>(a, 4096, st);
+    if (nvec <= 512) return launch_sq_nv<FMT, ROUND, 2, 4, 2, 4>(a, 1100, st);
+    if (nvec <= 1024) return launch_sq_nv<FMT, ROUND, 4, 4, 2, 8>(a, 192, st);
+    if (nvec <= 1536) return launch_sq_nv<FMT, ROUND, 6, 4, 3, 8>(a, 192, st);
+    if (nvec <= 1792) return launch_sq_nv<FMT, ROUND, 7, 4, 4, 8>(a, 192, st);
+    return launch_sq_nv<FMT, ROUND, 8, 4, 4, 8>(a, 192, st);
 }
 
 }  // namespace

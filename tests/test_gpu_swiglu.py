@@ -54,7 +54,7 @@ def _check(ops, oracle, device, x, fmt, rounding, want_out=True, want_codes=True
 @pytest.mark.parametrize("fmt,rounding", FMTS)
 @pytest.mark.parametrize("rows,half", [(64, 1024), (37, 5376), (9, 7168), (5, 14336), (3, 16384), (130, 2048),
                                        (2, 8), (17, 1000), (9, 13824),
-                                       # 1024 rows and more: the table form (s looked up per gate pattern)
+                                       # the two long ones: the table form (s looked up per gate pattern)
                                        (1024, 1024), (1061, 13824), (1030, 14336)])
 def test_swiglu_matches_oracle(ops, oracle, device, fmt, rounding, rows, half):
     _check(ops, oracle, device, _inputs(rows, half, seed=rows + half), fmt, rounding)
@@ -74,9 +74,9 @@ def test_codes_only_output_only_and_strided_rows(ops, oracle, device):
 
 
 def test_table_form_strided_rows(ops, oracle, device):
-    """1030 rows (the table form) read from a wider buffer and written into
+    """1030 long rows (the table form) read from a wider buffer and written into
     row slices of wider output and code buffers: bit-exact."""
-    half = 1024
+    half = 4104
     wide = _inputs(1030, 2 * half + 64, 8)
     x = wide[:, :2 * half]
     out_wide = torch.zeros(1030, half + 32, device=device, dtype=torch.bfloat16)
@@ -112,15 +112,15 @@ def test_special_values(ops, oracle, device):
     np.testing.assert_array_equal(bits16(out), oracle.swiglu(bits16(x)))
 
 
-@pytest.mark.parametrize("rows", [64, 1024])
+@pytest.mark.parametrize("rows", [64, 1024, 8192])
 def test_every_bf16_gate(ops, oracle, device, rows):
     """silu depends on the gate alone, so the 65536 bf16 gate values (NaNs,
     infinities, subnormals and both zeros included) with up = 1 cover it
     completely: y = bf16(silu(gate)) bit-exact against the oracle, whose exp
     is the IEEE-only restatement while the kernel uses the hardware exp2.
-    NaN gates must give NaN (the payload is not compared).  64 rows run the
-    direct form; 1024 rows the table form, whose device table this covers
-    entry by entry."""
+    NaN gates must give NaN (the payload is not compared).  64 rows and
+    1024 rows run the direct form; 8192 rows the table form, whose device table
+    this covers entry by entry."""
     gate = np.arange(65536, dtype=np.uint32).astype(np.uint16).reshape(rows, 65536 // rows)
     up = np.full(gate.shape, 0x3F80, dtype=np.uint16)  # bf16 1.0
     xb = np.concatenate([gate, up], axis=1)
@@ -198,9 +198,13 @@ def test_host_checks(ops, device):
 
 
 @pytest.mark.parametrize("fmt,rounding", FMTS)
-@pytest.mark.parametrize("rows,half", [(191, 1024), (192, 1024), (193, 4096), (515, 7168), (195, 8200), (261, 14336),
-                                       (197, 16384), (1, 16384), (33, 4104)])
+@pytest.mark.parametrize("rows,half", [(191, 4104), (192, 4104), (193, 4096), (515, 7168), (195, 8200), (261, 14336),
+                                       (197, 16384), (1, 16384), (33, 4104),
+                                       # one, two and four waves to a row, directly and by the table
+                                       (7, 8), (8191, 512), (8195, 504), (5, 520), (5119, 1024), (5121, 520),
+                                       (3, 1032), (4095, 1032), (4097, 2048), (1099, 4096), (1101, 2056)])
 def test_swiglu_rows_shared_by_waves(ops, oracle, device, fmt, rounding, rows, half):
-    """Both sides of the row count where the table form starts, ragged last
-    row groups, and row widths at the edges of each number of vectors per lane."""
+    """Both sides of the row counts where the table form starts, ragged last
+    row groups, and row widths at the edges of each number of waves per row and of
+    vectors per lane."""
     test_swiglu_matches_oracle(ops, oracle, device, fmt, rounding, rows, half)

@@ -563,10 +563,14 @@ __global__ __launch_bounds__(256) void tensor_quant_typed_kernel(const void* __r
 
 // Vector path (bf16, fp16 or fp32; K % 8 == 0, 16-byte aligned rows of x, 8-byte
 // aligned rows of q): the tensor is a list of 8-element vectors, vector p at row
-// p / (K / 8); FLAT (rows adjacent in x and q) skips the division.  Thread t of
-// workgroup b takes the vectors b * 256 + t + j * 256 * grid, several of them in
-// flight, so the work is even whatever the shape: a row per wave left 100 rows
-// on 25 CUs, and the elementwise typed form moved 2 bytes per load.  Grids of more
+// p / (K / 8); FLAT (rows adjacent in x and q) skips the division.  A workgroup takes
+// runs of 256 vectors, one per thread, several of them in flight, so the work is
+// even whatever the shape: a row per wave left 100 rows on 25 CUs, and the
+// elementwise typed form moved 2 bytes per load.  The runs in flight lie a grid
+// apart, or (BAND, tensors of more trips than one) side by side: four streams 4 MB
+// apart read slower than one (bf16 [8192, 5120] from HBM, a row per wave / apart / side
+// by side: both passes 37.6 / 39.2 / 36.8 us, quantize alone 24.4 / 25.1 / 22.2; [40960,
+// 5120] 197 / 211 / 196, 119 / 129 / 119).  Grids of more
 // than 8 workgroups are multiples of 8, so both passes read a vector on the same
 // XCD and pass 2 finds a tensor of up to about 30 MB in its L2.
 // Measured: amax 10.5 -> 5.0 and quantize 12.6 -> 8.4 us for fp16 [4090, 2048], 4.9 ->
@@ -655,6 +659,17 @@ struct TensorVec {  // 8 elements as loaded
     }
 };
 
+// First vector of this thread and the distance of its U vectors in flight; the next
+// trip is U grids of 256 vectors on.
+template <int U, bool BAND>
+struct VecRuns {
+    int64_t first, step, trip;
+    __device__ __forceinline__ VecRuns()
+        : first((int64_t)blockIdx.x * 256 * (BAND ? U : 1) + threadIdx.x),
+          step(BAND ? 256 : (int64_t)gridDim.x * 256),
+          trip((int64_t)gridDim.x * 256 * U) {}
+};
+
 // Element offset of vector p in a matrix of row stride ld.
 template <bool FLAT>
 __device__ __forceinline__ int64_t vec_offset(int64_t p, int64_t ld, uint32_t nvec) {
@@ -663,18 +678,18 @@ __device__ __forceinline__ int64_t vec_offset(int64_t p, int64_t ld, uint32_t nv
     return row * ld + ((uint32_t)p - row * nvec) * 8;
 }
 
-template <int IN, bool FLAT>
+template <int IN, bool FLAT, bool BAND>
 __global__ __launch_bounds__(256) void tensor_amax_vec_kernel(const void* __restrict__ x, int64_t ldx, uint32_t nvec,
                                                               int64_t total, float* __restrict__ partial) {
     constexpr int U = 4;
     __shared__ float red[4];
-    const int64_t step = (int64_t)gridDim.x * 256;
+    const VecRuns<U, BAND> runs;
     uint32_t m = 0;
-    for (int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x; p < total; p += U * step) {
+    for (int64_t p = runs.first; p < total; p += runs.trip) {
         TensorVec<IN> v[U];
 #pragma unroll
         for (int j = 0; j < U; ++j)  // past the end: the last vector again
-            v[j].load(x, vec_offset<FLAT>(p + j * step < total ? p + j * step : total - 1, ldx, nvec));
+            v[j].load(x, vec_offset<FLAT>(p + j * runs.step < total ? p + j * runs.step : total - 1, ldx, nvec));
 #pragma unroll
         for (int j = 0; j < U; ++j) m = v[j].amax_bits(m);
     }
@@ -684,20 +699,20 @@ __global__ __launch_bounds__(256) void tensor_amax_vec_kernel(const void* __rest
 }
 
 // Pass 2: U vectors per thread in flight, the first of them under the fold.
-template <int IN, int RND, bool FLAT, int U>
+template <int IN, int RND, bool FLAT, int U, bool BAND>
 __global__ __launch_bounds__(256) void tensor_quant_vec_kernel(const void* __restrict__ x, int64_t ldx, uint32_t nvec,
                                                                int64_t total, const float* __restrict__ partial,
                                                                int nparts, const float* __restrict__ static_scale,
                                                                int eager, uint8_t* __restrict__ q, int64_t ldq,
                                                                float* __restrict__ scale_out) {
     __shared__ float red[4];
-    const int64_t step = (int64_t)gridDim.x * 256;
-    int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const VecRuns<U, BAND> runs;
+    int64_t p = runs.first;
     TensorVec<IN> v[U];
     auto load = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < U; ++j)
-            v[j].load(x, vec_offset<FLAT>(p + j * step < total ? p + j * step : total - 1, ldx, nvec));
+            v[j].load(x, vec_offset<FLAT>(p + j * runs.step < total ? p + j * runs.step : total - 1, ldx, nvec));
     };
     load();
     const TensorQuant tq = tensor_scale(partial, nparts, static_scale, eager ? RND : 0, red, scale_out);
@@ -706,12 +721,12 @@ __global__ __launch_bounds__(256) void tensor_quant_vec_kernel(const void* __res
 #pragma unroll
         for (int j = 0; j < U; ++j) u[j] = v[j];
         const int64_t p0 = p;
-        p += U * step;
+        p += runs.trip;
         if (p < total) load();
 #pragma unroll
         for (int j = 0; j < U; ++j)
-            if (p0 + j * step < total)
-                *reinterpret_cast<uint2*>(q + vec_offset<FLAT>(p0 + j * step, ldq, nvec)) =
+            if (p0 + j * runs.step < total)
+                *reinterpret_cast<uint2*>(q + vec_offset<FLAT>(p0 + j * runs.step, ldq, nvec)) =
                     u[j].template pack8<RND>(tq);
     }
 }
@@ -731,13 +746,19 @@ int64_t tensor_vectors(const void* x, int64_t ldx, int64_t rows, int64_t k, cons
     return rows * nvec;
 }
 
-template <int IN, int RND, bool FLAT, int U>
+template <int IN, int RND, bool FLAT, int U, bool BAND>
 hipError_t launch_tensor_vec_u(const void* x, int64_t ldx, int64_t k, int64_t total, int64_t parts, int64_t blocks,
                                const float* static_scale, bool eager, float* partial, uint8_t* q, int64_t ldq,
                                float* scale_out, hipStream_t st) {
-    hipLaunchKernelGGL((tensor_quant_vec_kernel<IN, RND, FLAT, U>), dim3((unsigned)blocks), dim3(256), 0, st, x, ldx,
-                       (uint32_t)(k / 8), total, (const float*)partial, (int)parts, static_scale, (int)eager, q, ldq,
-                       scale_out);
+    if (!static_scale) {
+        hipLaunchKernelGGL((tensor_amax_vec_kernel<IN, FLAT, BAND>), dim3((unsigned)parts), dim3(256), 0, st, x, ldx,
+                           (uint32_t)(k / 8), total, partial);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL((tensor_quant_vec_kernel<IN, RND, FLAT, U, BAND>), dim3((unsigned)blocks), dim3(256), 0, st, x,
+                       ldx, (uint32_t)(k / 8), total, (const float*)partial, (int)parts, static_scale, (int)eager, q,
+                       ldq, scale_out);
     return hipGetLastError();
 }
 
@@ -750,21 +771,16 @@ hipError_t launch_tensor_vec(const void* x, int64_t ldx, int64_t rows, int64_t k
     int64_t parts = rows < kTensorBlocks ? rows : kTensorBlocks;
     if (parts > chunks) parts = chunks;
     if (parts > 8) parts &= ~(int64_t)7;
-    if (!static_scale) {
-        hipLaunchKernelGGL((tensor_amax_vec_kernel<IN, FLAT>), dim3((unsigned)parts), dim3(256), 0, st, x, ldx,
-                           (uint32_t)(k / 8), total, partial);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-    }
     // Pass 2: up to two chunks per workgroup while that fits the chip at once, then
-    // half as many workgroups of four in flight.
+    // half as many workgroups of four in flight, side by side.
     const int64_t per = (chunks + kTensorChunks - 1) / kTensorChunks;
     int64_t blocks = per <= 2 ? (chunks + per - 1) / per : kTensorChunks / 2;
     blocks = (blocks + 7) & ~(int64_t)7;
-#define H3Q_U(U) launch_tensor_vec_u<IN, RND, FLAT, U>(x, ldx, k, total, parts, blocks, static_scale, eager, partial, q, ldq, scale_out, st)
-    if (per <= 1) return H3Q_U(1);
-    if (per <= 2) return H3Q_U(2);
-    return H3Q_U(4);
+#define H3Q_U(U, BAND) \
+    launch_tensor_vec_u<IN, RND, FLAT, U, BAND>(x, ldx, k, total, parts, blocks, static_scale, eager, partial, q, ldq, scale_out, st)
+    if (per <= 1) return H3Q_U(1, false);
+    if (per <= 2) return H3Q_U(2, false);
+    return H3Q_U(4, true);
 #undef H3Q_U
 }
 

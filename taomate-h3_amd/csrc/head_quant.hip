@@ -29,7 +29,8 @@
 // that a wavefront needs few registers and many wavefronts share a SIMD:
 // their loads and their arithmetic then overlap.  Traffic per element: 2
 // bytes (pass 1) + 2 + 1 bytes (pass 3); algorithmic 3 bytes.  Up to 256 token
-// chunks the fold of pass 2 runs inside pass 3 instead (two launches).
+// chunks and 32 heads per column group the fold of pass 2 runs inside pass 3 instead
+// (two launches).
 #include "h3q_common.hpp"
 #include "h3q_kernels.hpp"
 #include "row_quant.hpp"  // pk_abs_max, amax_from_packed
@@ -38,7 +39,9 @@ namespace h3q {
 
 namespace {
 
-constexpr int kFoldChunks = 256;  // token chunks up to which pass 3 folds the partial maxima itself
+// Pass 3 folds the partial maxima itself up to these token chunks, heads in a column
+// group and column groups that a head lies in (see head_quant_kernel).
+constexpr int kFoldChunks = 256, kFoldHeads = 32, kFoldGroups = 2;
 
 struct HeadQuantShape {
     int64_t batch, seq, heads, head_dim;
@@ -197,14 +200,18 @@ __global__ __launch_bounds__(256) void head_scale_kernel(const float* __restrict
 }
 
 // Pass 3.  blockIdx.x = (b * G + g) * C + c.
-// FOLD (G <= kFoldChunks): pass 2 happens here.  A workgroup folds the partials
-// of the heads in its column group (a head lies in one or two groups; a wave
-// takes four neighbouring heads at a time, all their loads and its first row of
-// x in flight together) into LDS, and chunk 0 of each group stores the scales.  Dynamic LDS: H words.  The fold reads 4 G
-// bytes per head and workgroup from the L2, which costs less than the launch it
-// saves: 28.8 -> 24.7 us in all at [1, 3121, 56, 128], 12.8 -> 11.3 us at
-// [1, 300, 28, 64] (kernel times); with more chunks the fold grows (G = 512: 57 KB per
-// workgroup), so longer inputs keep the pass of its own.
+// FOLD: pass 2 happens here.  A workgroup folds the partials of the heads in its
+// column group (a wave takes four neighbouring heads at a time, all their loads and
+// its first row of x in flight together) into LDS, and chunk 0 of each group stores
+// the scales.  Dynamic LDS: H words.  The fold reads 4 G bytes per head and
+// workgroup from the L2, two batches of four heads a wave at most.  That costs less
+// than the launch it saves (us, a pass of its own / folded, x from HBM): 28.8 / 24.7 at
+// [1, 3121, 56, 128] (kernel times), 20.8 / 19.3 at [1, 2048, 56, 128], 12.2 / 11.4 at [1,
+// 300, 28, 64], 15.1 / 14.5 at [1, 4096, 28, 64].  Each further batch is another round trip
+// in every workgroup, and so is each further column group of a wide head: 40 heads of 64 in a group
+// 12.2 / 12.6 at 64 tokens and even from 1024 on, 56 14.3 / 15.6 at 300 and 20.7 / 21.4 at
+// 4096, 256 of 16 15.7 / 28.2, 448 of 8 14.8 / 38.6.  With more chunks the fold grows too
+// (G = 512: 57 KB per workgroup).  Those keep the pass of its own.
 template <class IO, int NS, bool FOLD>
 __global__ __launch_bounds__(256) void head_quant_kernel(const uint16_t* __restrict__ x, HeadQuantShape sh,
                                                          const float* __restrict__ partial,
@@ -333,7 +340,11 @@ hipError_t launch_head_quant_ns(const uint16_t* x, const HeadQuantShape& sh, flo
     hipLaunchKernelGGL((head_amax_kernel<IO, NS>), grid, blk, (size_t)sh.heads * 4, st, x, sh, partial);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    if (sh.chunks <= kFoldChunks) {
+    // Heads that a column group of 64 NS positions holds positions of, and groups of a head, at most.
+    const int64_t group = 64 * NS * (sh.head_dim % 8 == 0 ? 8 : 1);
+    const int64_t heads = (group + sh.head_dim - 2) / sh.head_dim + 1, groups = (sh.head_dim + group - 2) / group + 1;
+    if (sh.chunks <= kFoldChunks && (heads < sh.heads ? heads : sh.heads) <= kFoldHeads &&
+        (groups < sh.groups ? groups : sh.groups) <= kFoldGroups) {
         hipLaunchKernelGGL((head_quant_kernel<IO, NS, true>), grid, blk, (size_t)sh.heads * 4, st, x, sh,
                            (const float*)partial, scales, q);
         return hipGetLastError();

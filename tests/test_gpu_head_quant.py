@@ -217,3 +217,11 @@ def test_scales_folded_by_the_quantize_pass(ops, oracle, device, shape):
     rq, rs = oracle.quant_per_head_e4m3(bits16(x).reshape(shape))
     np.testing.assert_array_equal(bits8(codes).reshape(-1), np.asarray(rq).reshape(-1).view(np.uint8))
     np.testing.assert_array_equal(scales.cpu().numpy().reshape(-1), np.asarray(rs).reshape(-1))
+
+
+@pytest.mark.parametrize("shape", [(1, 300, 32, 64), (1, 300, 33, 64), (1, 40, 64, 32), (2, 100, 448, 8),
+                                   (1, 70, 3, 1001), (1, 40, 1, 8200), (1, 33, 31, 100)])
+def test_scales_of_many_or_wide_heads(ops, oracle, device, shape):
+    """Both sides of the heads per column group and of the column groups per head
+    up to which the quantize pass folds the partial maxima."""
+    test_scales_folded_by_the_quantize_pass(ops, oracle, device, shape)

@@ -47,6 +47,10 @@ StreamChoice best_stream_tile(int64_t m, int64_t n, int64_t k) {
 bool stream_takes(const GemmArgs& a) {
     // 16-byte output pieces and 32-bit block-relative offsets.
     if (a.n % 8 || a.ldo % 8 || (uintptr_t)a.out % 16 || a.k < 128) return false;
+    // The bias comes in by LDS copies of whole dwords.  The per-tile kernels, whose
+    // calls with a K tail, binary16 output or few rows and an adapter come here, read
+    // it element by element and keep those with a bias at an odd element.
+    if ((uintptr_t)a.bias % 4) return false;
     if (a.lora_t && (a.out_f16 || a.lora_rank > 128)) return false;
     return 256 * a.k < (int64_t(1) << 30);
 }

@@ -127,3 +127,20 @@ def test_stream_k_tail_at_any_size(ops, oracle, device, m, n, k):
     rqw, rsw = oracle.quant_rows(bits16(w), "int8", "div")
     ref = oracle.epilogue(oracle.gemm_i8_i32_fast(rqa, rqw), rsa, rsw, None)
     np.testing.assert_array_equal(bits16(out), ref)
+
+
+@pytest.mark.parametrize("m,n,k", [(200, 264, 272), (300, 520, 1040)])
+def test_bias_at_an_odd_element(ops, oracle, device, m, n, k):
+    """A bias that starts at an odd 2-byte element takes the kernel that reads it element by element."""
+    print(f"odd bias {m}x{n}x{k}", flush=True)
+    x, w, qa, sa, qw, sw = _operands(ops, device, m, n, k, "int8", False, False)
+    packed = (torch.randn(n + 1, generator=torch.Generator().manual_seed(5)) * 0.1).to(torch.float16)
+    bias = packed.to(device)[1:]
+    assert bias.data_ptr() % 4 == 2
+    out = ops.scaled_mm(qa, qw, sa, sw, bias=bias, out_dtype=torch.float16)
+    torch.cuda.synchronize()
+    acc = oracle.gemm_i8_i32_fast(*(oracle.quant_rows(bits16(t), "int8", r)[0] for t, r in ((x, "rcp"), (w, "div"))))
+    v = (sw.cpu().numpy().astype(np.float64) * acc.astype(np.float64)).astype(np.float32).astype(np.float64)
+    exact = sa.cpu().numpy().astype(np.float64)[:, None] * v + packed[1:].double().numpy()
+    ref = exact.astype(np.float32).astype(np.float16)  # one rounding each: s_w * acc, the fma
+    np.testing.assert_array_equal(out.cpu().numpy().view(np.uint16), ref.view(np.uint16))

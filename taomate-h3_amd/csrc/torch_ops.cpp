@@ -134,7 +134,8 @@ Opt lora_down(const Tensor& x, const Tensor& lora_a, Opt out, int64_t stream) {
     if (!x.is_cuda() || !on(lora_a, x) || !rows_2d(x, at::kBFloat16) || !rows_2d(lora_a, at::kBFloat16)) return std::nullopt;
     const int64_t m = x.size(0), k = x.size(1), rank = lora_a.size(0);
     if (m == 0 || lora_a.size(1) != k) return std::nullopt;
-    if (out && !(on(*out, x) && rows_2d(*out, at::kBFloat16))) return std::nullopt;
+    if (out && !(on(*out, x) && rows_2d(*out, at::kBFloat16) && out->size(0) >= m && out->size(1) >= rank))
+        return std::nullopt;
     if (!out) out = empty(x, {m, rank}, at::kBFloat16);
     const int64_t bytes = h3q_lora_down_workspace_bytes(m, k, rank);
     int rc;

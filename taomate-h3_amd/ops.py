@@ -594,6 +594,8 @@ def lora_down(x: torch.Tensor, lora_a: torch.Tensor, *, out: torch.Tensor | None
     if out is None:
         out = torch.empty((m, rank), device=x.device, dtype=torch.bfloat16)
     _rows_2d("lora_down out", out, torch.bfloat16)
+    if out.shape[0] < m or out.shape[1] < rank:
+        raise ValueError(f"lora_down: out shape {tuple(out.shape)} does not hold {(m, rank)}")
     if m == 0:
         return out
     # Few rows: the library splits K and needs a binary32 workspace for the

@@ -141,8 +141,9 @@ def test_native_wrappers_equal_the_python_ones(ops, device, monkeypatch):
 
 def test_native_wrappers_refuse_what_the_python_ones_refuse(ops, device, monkeypatch):
     """Row counts and formats below zero, and a residual gate without its
-    tensors, are no way to say "not given": the same error as without the
-    native wrapper."""
+    tensors, are no way to say "not given", and an output that does not hold the
+    result is refused before the launch: the same error as without the native
+    wrapper."""
     x = activations(37, 512, seed=3).to(device)
     q, s = ops.quant_rows(x, ops.FMT_INT8)
     one = torch.ones(1, device=device)
@@ -160,6 +161,8 @@ def test_native_wrappers_refuse_what_the_python_ones_refuse(ops, device, monkeyp
         "norm gate without a branch": lambda: norm(residual_gate=(None, table, torch.empty_like(x))),
         "norm gate without a table": lambda: norm(residual_gate=(x, None, torch.empty_like(x))),
         "swiglu format": lambda: ops.swiglu_quant(x, fmt=-1, out=True),
+        "down rows": lambda: ops.lora_down(x, x[:16], out=torch.empty(36, 16, device=device, dtype=torch.bfloat16)),
+        "down rank": lambda: ops.lora_down(x, x[:16], out=torch.empty(37, 8, device=device, dtype=torch.bfloat16)),
     }
     for name, call in calls.items():
         print(name, flush=True)

@@ -4,6 +4,8 @@ here and not only in a measurement."""
 
 from __future__ import annotations
 
+import random
+
 import pytest
 
 from _util import gemm_plan
@@ -42,3 +44,26 @@ def test_few_rows_with_an_adapter():
     assert gemm_plan(16, 5120, 5120, b_tiled=True, rank=64)[0] == STREAM
     assert gemm_plan(128, 2048, 2048, rank=8)[0] == STREAM
     assert gemm_plan(16, 5116, 5120, b_tiled=True, rank=64)[0] == "per tile"
+
+
+@pytest.mark.parametrize("m,n,k,split", [(5130, 3336, 1536, 3072), (1030, 16904, 2048, 13056),
+                                         (4362, 4104, 1536, -3840), (2049, 8712, 1536, -1792),
+                                         (4608, 4096, 1024, -4096), (5130, 4104, 1024, 0), (8192, 15360, 5120, 0)])
+def test_calls_in_two_launches(m, n, k, split):
+    """First columns, or (negative) first rows, of the four-wave part; 0: one launch."""
+    plan = gemm_plan(m, n, k, a_tiled=True, b_tiled=True)
+    assert plan[0] == ("split" if split else "four waves") and plan[2] == split
+
+
+def test_the_layouts_do_not_decide_above_128_rows():
+    """Nor at any row count with an adapter: such a call gives the same bits in every layout."""
+    rng = random.Random(7)
+    for _ in range(2000):
+        m = round(129 * (20000 / 129) ** rng.random())
+        n, k = 8 * rng.randint(1, 2000), 128 * rng.randint(2, 110)
+        rank = rng.choice((0, 0, 64))
+        plans = {gemm_plan(m, n, k, a_tiled=a, b_tiled=b, rank=rank)
+                 for a in (False, True) for b in (False, True)}
+        assert len(plans) == 1, (m, n, k, rank, plans)
+        few = 1 + m % 128
+        assert gemm_plan(few, n, k, rank=64) == gemm_plan(few, n, k, b_tiled=True, rank=64)

@@ -149,8 +149,8 @@ def _assert_fp8_f16_close(oracle, got_bits, rqa, rsa, rqw, rsw, bias_bits):
         assert same >= 0.99, same
 
 
-# Shapes by kernel: four-wave (512 x 1024 x 1024), persistent (n % 8 != 0),
-# tile (k % 128 != 0), weight-streaming (m <= 128).
+# Shapes by kernel: streaming tiles (512 x 1024 x 1024 and the K tail of 300 x 200 x
+# 1040), per tile (n % 8 != 0), few rows (m <= 128); four waves in test_gpu_gemm_tiles.
 _F16_SHAPES = [(512, 1024, 1024), (300, 1004, 1024), (300, 200, 1040), (16, 512, 1024), (100, 96, 256)]
 
 

@@ -195,7 +195,9 @@ def test_c5_int8_full_size_bit_exact(ops, oracle, device, a_tiled):
 @pytest.mark.parametrize("per_tensor", [False, True])
 def test_more_tiles_than_workgroups(ops, oracle, device, fmt, per_tensor):
     """m=4608, n=4096, k=1024 with tiled weights and bias: 288 output tiles,
-    more than the persistent grid, so 32 workgroups run a second tile.
+    more than the persistent grid: 256 of them in one round of the four-wave
+    kernel, the last two tile-rows over smaller tiles (in one launch with a second
+    round: test_gpu_gemm_tiles).
     int8: every row bit-exact.  e4m3: whole tile-rows 0, 8 and 17 and the
     boundaries against the instruction model.  Per-row and per-tensor scales."""
     m, n, k = 4608, 4096, 1024
@@ -227,7 +229,7 @@ def test_more_tiles_than_workgroups(ops, oracle, device, fmt, per_tensor):
 
 def test_ragged_large_m_tiled_activations(ops, oracle, device):
     """A ragged M (not a multiple of 16 or 256) with tiled activations and
-    tiled weights through the four-wave GEMM, int8: every output bit-exact."""
+    tiled weights through 112 x 128 streaming tiles, int8: every output bit-exact."""
     m, n, k = 1000, 3000, 1024
     x = activations(m, k, seed=17, outlier_channels=5)
     w = weights(n - 8, k, seed=18)            # n = 2992: a partial last tile column
@@ -336,7 +338,8 @@ def test_h3_production_shapes_int8(ops, oracle, device, name, m, n, k):
     fc1 N = 14336, K = 5376 = 42 k-steps of 128; M per Ulysses rank from
     H3/streaming/geometry.py:173-200, a multiple of 16 but not of 256):
     per-token int8 activations (vLLM form) in the tiled layout, tiled int8
-    weights, no bias, as quant_activations_for feeds the four-wave GEMM.
+    weights, no bias, as quant_activations_for feeds the GEMMs above 128 rows
+    (592 rows: streaming tiles; 2640: four waves and streaming tiles).
     Codes and bf16 outputs bit-exact on every 256-row tile-row's sampled rows,
     the ragged last tile-row whole."""
     print(f"H3 {name}: {m}x{n}x{k} int8", flush=True)

@@ -343,14 +343,14 @@ def test_lora_down_slice_counts(ops, oracle, device, m, k, rank):
     test_lora_down_split_over_k(ops, oracle, device, m, k, rank)
 
 
-@pytest.mark.parametrize("m,a_tiled", [(512, False), (512, True), (64, False), (16, True)])
+@pytest.mark.parametrize("m,a_tiled", [(512, False), (512, True), (64, False), (16, True), (16400, True)])
 def test_fp8_nan_codes_propagate(ops, device, m, a_tiled):
     """A NaN code (0x7F / 0xFF in e4m3fn) in an activation row makes exactly
     that output row NaN, and one in a weight row exactly that output column,
     as exact arithmetic (and the reference's torch._scaled_mm) gives; every
-    other element equals the NaN-free call bit for bit.  Large M (four-wave
-    kernel, row-major or tiled activations) and M <= 128 (weight-streaming
-    kernel)."""
+    other element equals the NaN-free call bit for bit.  Streaming tiles
+    (512 rows, row-major or tiled activations), few rows, and the four-wave kernel
+    (16400 rows)."""
     from _util import to_tiled
 
     k, n = 1024, 768

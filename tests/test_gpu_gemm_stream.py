@@ -1,8 +1,9 @@
-"""The weight-streaming GEMM over chip-filling tiles (gemm_stream.hpp), at the
-sizes where a tile, ring or reduction can go wrong: the smallest and ragged row
-counts of every tile height, ragged column counts, fewer k-tiles than the
-rings hold, k-tiles that do not divide among the K groups, a K tail (row-major
-only), both layouts of both operands, binary16 output and the LoRA epilogue.
+"""The weight-streaming GEMM over chip-filling tiles (gemm_stream.hpp; some calls of
+up to 128 rows take the few-rows kernels instead), at the sizes where a ring or a
+reduction can go wrong: one row past 64, 80, 96, 112 and 128, ragged column counts,
+fewer k-tiles than the rings hold, k-tiles that do not divide among the K groups, a K
+tail (row-major only), both layouts of both operands, binary16 output and the LoRA
+epilogue.  These sizes take the smaller tiles; test_gpu_gemm_tiles runs every tile.
 int8 against the oracle bit for bit, e4m3 against the instruction model to the
 bound of test_gpu_gemm."""
 
@@ -26,8 +27,8 @@ def _operands(ops, device, m, n, k, fmt, a_tiled, b_tiled):
     return x, w, qa, sa.reshape(-1), qw, sw.reshape(-1)
 
 
-# (m, n, k): one row past a tile of 64, 80, 96, 112 and 128 rows and exact ones,
-# on every tile width; K of 1, 2, 3, 5 and 9 k-tiles; n = 8 alone and past a tile.
+# (m, n, k): one row past 64, 80, 96, 112 and 128 rows and exact ones; K of 1, 2, 3, 5
+# and 9 k-tiles; n = 8 alone and past a tile.
 _CASES = [(33, 8200, 256, True, True), (65, 264, 128, True, True), (128, 520, 384, False, True),
           (129, 264, 256, True, True), (161, 1032, 640, True, True), (300, 8, 1152, False, True),
           (337, 2056, 256, True, True), (449, 4104, 384, False, True), (700, 3592, 640, True, True),

@@ -2,10 +2,11 @@
 output strides: every output bit-exact against the oracle epilogue of the
 exact int32 accumulators (the int8 W8A8 linear, H3/inference/w8a8.py:179-186).
 
-The shapes cover the weight-streaming kernel (m <= 128), the four-wave kernel
-with whole and half tiles, and the row-major fallbacks (k not a multiple of
-128); n and m are ragged against every tile size, and some outputs are
-strided views whose rows do not allow vector stores."""
+The shapes cover the few-rows kernels (m <= 128), the smallest streaming tiles
+(with a K tail too) and the per-tile fallbacks (n or the output's row stride not a
+multiple of 8); n and m are ragged against every tile size, and some outputs are
+strided views whose rows do not allow vector stores.  The larger streaming tiles
+and the four-wave kernel: test_gpu_gemm_tiles."""
 
 from __future__ import annotations
 
@@ -32,7 +33,7 @@ def _cases(count: int = 32, seed: int = 20261202):
         if m * n * k > 3e8:
             continue
         pad = rng.choice([0, 0, 3, 8])
-        if a_tiled and m > 128:  # tiled activations past the skinny rows: the four-wave kernel's shapes only
+        if a_tiled and m > 128:  # tiled activations above 128 rows: the shapes that take them
             n, k, pad = (n + 7) // 8 * 8, max(k, 256), pad // 8 * 8
         out.append((m, n, k, a_tiled, b_tiled, rng.random() < 0.5, pad))
     return out

@@ -158,7 +158,7 @@ __device__ __forceinline__ void load_row(const uint16_t* __restrict__ x, int64_t
 // of X overlap the stores.
 __device__ __forceinline__ int img_chunk(int c, int r) { return (c & ~15) | ((c & 15) ^ ((r & 1) | ((r >> 1) << 2))); }
 
-template <int FMT, int ROUND, int NV, bool PREFETCH>
+template <int FMT, int ROUND, int NV>
 __global__ __launch_bounds__(512) void quant_rows_tiled_img_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                                    int64_t rows, int k, uint8_t* __restrict__ q,
                                                                    int64_t row0, float* __restrict__ scales) {
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(512) void quant_rows_tiled_img_kernel(const uint16_
     auto load = [&](int64_t un, auto& dst) __attribute__((always_inline)) {
         load_row<NV>(x, ldx, 8 * un + r, 8 * un + r < rows ? nvec : 0, lane, dst);
     };
-    uint4 v[NV], vn[PREFETCH ? NV : 1];
+    uint4 v[NV], vn[NV];
     int64_t u = blockIdx.x;
     if (u < units) load(u, v);
     while (u < units) {
@@ -202,9 +202,7 @@ __global__ __launch_bounds__(512) void quant_rows_tiled_img_kernel(const uint16_
             }
         }
         const int64_t un = u + gridDim.x;
-        if constexpr (PREFETCH) {
-            if (un < units) load(un, vn);
-        }
+        if (un < units) load(un, vn);
         __syncthreads();
         // Read-back: slot t = ((s * 2 + h) * 4 + qq) * 8 + rr holds row rr,
         // codes 128 s + 32 qq + 16 h .. + 15.
@@ -221,12 +219,8 @@ __global__ __launch_bounds__(512) void quant_rows_tiled_img_kernel(const uint16_
             *reinterpret_cast<uint4*>(qb + (int64_t)s * 2048 + h * 1024 + (8 * half + rr + 16 * qq) * 16) = val;
         }
         __syncthreads();  // the image is written again by the next unit
-        if constexpr (PREFETCH) {
 #pragma unroll
-            for (int i = 0; i < NV; ++i) v[i] = vn[i];
-        } else if (un < units) {
-            load(un, v);
-        }
+        for (int i = 0; i < NV; ++i) v[i] = vn[i];
         u = un;
     }
 }
@@ -297,31 +291,23 @@ static hipError_t launch_rows_wide(const uint16_t* x, int64_t ldx, int64_t rows,
     return hipGetLastError();
 }
 
-template <int FMT, int ROUND, int NV, bool PREFETCH>
-static hipError_t launch_rows_tiled_img_cfg(const uint16_t* x, int64_t ldx, int64_t rows, int64_t k, uint8_t* q,
-                                            int64_t row0, float* scales, int per_cu, hipStream_t st) {
-    const int64_t units = (rows + 7) / 8;
-    const int64_t img_bytes = 8 * ((k + 255) & ~int64_t(255));
-    const int64_t cap = 256 * (int64_t)per_cu;
-    const int64_t grid = units < cap ? units : cap;
-    // Images above 64 KiB (K > 8192) need the kernel's dynamic LDS limit raised.
-    static const hipError_t lds_limit = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&quant_rows_tiled_img_kernel<FMT, ROUND, NV, PREFETCH>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, 8 * ((512 * NV + 255) & ~255));
-    if (lds_limit != hipSuccess) return lds_limit;
-    hipLaunchKernelGGL((quant_rows_tiled_img_kernel<FMT, ROUND, NV, PREFETCH>), dim3((unsigned)grid), dim3(512),
-                       (size_t)img_bytes, st, x, ldx, rows, (int)k, q, row0, scales);
-    return hipGetLastError();
-}
-
 template <int FMT, int ROUND, int NV>
 static hipError_t launch_rows_tiled_img(const uint16_t* x, int64_t ldx, int64_t rows, int64_t k, uint8_t* q,
                                         int64_t row0, float* scales, hipStream_t st) {
     // Workgroups of 8 waves: two per CU while the image (8 W bytes) and two
     // row register sets per lane (128 VGPRs) fit twice, else one.
+    const int64_t units = (rows + 7) / 8;
     const int64_t img_bytes = 8 * ((k + 255) & ~int64_t(255));
-    const int per_cu = (NV <= 12 && img_bytes <= 80 * 1024) ? 2 : 1;
-    return launch_rows_tiled_img_cfg<FMT, ROUND, NV, true>(x, ldx, rows, k, q, row0, scales, per_cu, st);
+    const int64_t cap = (NV <= 12 && img_bytes <= 80 * 1024) ? 512 : 256;
+    const int64_t grid = units < cap ? units : cap;
+    // Images above 64 KiB (K > 8192) need the kernel's dynamic LDS limit raised.
+    static const hipError_t lds_limit = hipFuncSetAttribute(
+        reinterpret_cast<const void*>(&quant_rows_tiled_img_kernel<FMT, ROUND, NV>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, 8 * ((512 * NV + 255) & ~255));
+    if (lds_limit != hipSuccess) return lds_limit;
+    hipLaunchKernelGGL((quant_rows_tiled_img_kernel<FMT, ROUND, NV>), dim3((unsigned)grid), dim3(512),
+                       (size_t)img_bytes, st, x, ldx, rows, (int)k, q, row0, scales);
+    return hipGetLastError();
 }
 
 template <int FMT, int ROUND>

@@ -65,6 +65,25 @@ double four_wave_cost(const GemmArgs& a) {
     return 8.0 + a.k / 64.0 * (0.68 * rounds + last);
 }
 
+// The same of the sixteen-wave kernels (gemm.hip), which take a K that is not a
+// multiple of 128: 128-byte k-tiles of 1.75 us in a full round of 256 x 256 tiles,
+// 1.13 us plus up to 0.8 by its tiles in the last one.
+double sixteen_wave_cost(const GemmArgs& a) {
+    const int64_t tiles = ceil_div(a.m, 256) * ceil_div(a.n, 256), ktiles = ceil_div(a.k, 128);
+    const int64_t rounds = tiles / kCus, rem = tiles % kCus;
+    const double last = rem == 0 ? 0.0 : 1.13 + 0.8 * rem / kCus;
+    return 11.0 * ceil_div(tiles, kCus) + ktiles * (1.75 * rounds + last);
+}
+
+// The streaming kernel with such a K, over its cost with tiled operands: against the
+// persistent sixteen-wave kernel, its binary16 form and its form with an adapter.
+// Measured on 1668 calls (192 .. 16384 rows, N 256 .. 5376, K 144 .. 4112): of 567 that
+// go to the sixteen-wave kernels almost all are faster there, up to 30% (3500 x 3520 x
+// 4112 binary16 65.6 against 80.9 us, with an adapter 65.1 / 84.2, 16384 x 4096 x 624 bf16
+// 84.0 / 103.5); those left are up to 3.8 times faster here (600 x 3520 x 1040 21.3 / 11.0,
+// 2600 x 256 x 4112 49.7 / 14.1), and 27 of them up to 10% slower.
+double tail_factor(const GemmArgs& a) { return a.lora_t ? 1.72 : (a.out_f16 ? 1.68 : 1.54); }
+
 // Whether the streaming tiles are the faster ones for M <= 128 rows, decided on
 // weights that come from HBM, as a step reads those of each layer (measured on
 // about 900 calls, N 512 .. 16384, K 256 .. 13824, both weight states; below, HBM
@@ -113,11 +132,7 @@ int stream_tile(const GemmArgs& a) {
     if (!stream_takes(a)) return 0;
     const StreamChoice best = best_stream_tile(a.m, a.n, a.k);
     if (a.m > kSkinnyMaxM) {
-        // K that is not a multiple of 128 would take the 16-wave kernel, slower in all
-        // of 35 calls of 132 .. 15049 rows, K 272 .. 4064 and N 256 .. 3520: 171 x 272 x
-        // 3824 55 -> 21 us, 11659 x 672 x 3488 205 -> 99, 12403 x 3296 x 1984 200 -> 133,
-        // 13191 x 2080 x 448 58 -> 54 (per-tensor binary16 linears, quantizer included).
-        if (a.k % 128) return best.tile;
+        if (a.k % 128) return tail_factor(a) * best.cost - 2.0 < sixteen_wave_cost(a) ? best.tile : 0;
         // Against the four-wave kernel: 0.78 keeps the calls that gain in both weight
         // states (Infinity Cache, HBM) and both layouts; of those left out the
         // best gained 8% in one state and lost 3% in the other.

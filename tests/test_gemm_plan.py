@@ -55,6 +55,17 @@ def test_calls_in_two_launches(m, n, k, split):
     assert plan[0] == ("split" if split else "four waves") and plan[2] == split
 
 
+@pytest.mark.parametrize("m,n,k,f16,rank,kernel", [
+    (600, 3520, 1040, True, 0, STREAM), (2600, 256, 4112, False, 0, STREAM), (4400, 4096, 2064, False, 64, STREAM),
+    (3500, 3520, 4112, True, 0, "per tile"), (3500, 3520, 4112, False, 64, "per tile"),
+    (16384, 4096, 624, False, 0, "per tile"), (9000, 3520, 2064, False, 0, "per tile"),
+    (12800, 2304, 1040, True, 0, "per tile"), (129, 8, 144, False, 0, STREAM)])
+def test_k_tails_above_128_rows(m, n, k, f16, rank, kernel):
+    """Row-major calls with a K that is not a multiple of 128: streaming tiles while
+    the 256 x 256 tiles of the sixteen-wave kernels leave most of the chip idle."""
+    assert gemm_plan(m, n, k, f16=f16, rank=rank)[0] == kernel
+
+
 def test_the_layouts_do_not_decide_above_128_rows():
     """Nor at any row count with an adapter: such a call gives the same bits in every layout."""
     rng = random.Random(7)

@@ -119,7 +119,8 @@ def test_stream_f16_output(ops, oracle, device, m, n, k):
 
 @pytest.mark.parametrize("m,n,k", [(129, 8, 144), (2600, 1040, 272), (4400, 2056, 656), (130, 4104, 4080)])
 def test_stream_k_tail_at_any_size(ops, oracle, device, m, n, k):
-    """K that is not a multiple of 128 takes this kernel above 128 rows whatever the sizes."""
+    """K that is not a multiple of 128 above 128 rows, at sizes on both sides of the
+    line to the sixteen-wave kernels."""
     print(f"stream K tail {m}x{n}x{k}", flush=True)
     x, w, qa, sa, qw, sw = _operands(ops, device, m, n, k, "int8", False, False)
     out = ops.scaled_mm(qa, qw, sa, sw)

@@ -113,3 +113,10 @@ def test_four_waves(ops, oracle, device, m, n, k, form):
     """One launch of 256 x 256 tiles, ragged in both directions; 357 of them on 256
     workgroups, and fewer tiles than workgroups."""
     _check(ops, oracle, device, m, n, k, form, ("four waves", (0, 0)))
+
+
+@pytest.mark.parametrize("form", ["int8 rows", "e4m3 rows per tensor", "f16", "e4m3 rows adapter"])
+@pytest.mark.parametrize("m,n,k", [(3500, 4104, 656), (6200, 2056, 1040)])
+def test_k_tail_per_tile(ops, oracle, device, m, n, k, form):
+    """A K tail at sizes that fill the chip with 256 x 256 tiles: the sixteen-wave kernels."""
+    _check(ops, oracle, device, m, n, k, form, ("per tile", (0, 0)))

@@ -198,8 +198,8 @@ int h3q_swiglu_quant(const void* x, int64_t ldx, int64_t rows, int64_t half, voi
  * batch == 0 or heads == 0 is a no-op; seq == 0 or head_dim == 0 is
  * H3Q_ERR_INVALID (an empty reduction, as torch's amax); heads <= 4096.
  * head_dim % 8 == 0 with a 16-byte aligned x and 8-byte aligned codes takes
- * the vector path; anything else runs element by element.  Two kernels:
- * per-chunk head maxima, then fold + quantize.
+ * the vector path; anything else runs element by element.  Two kernels
+ * (per-chunk head maxima, then fold + quantize), or three for many chunks or heads.
  */
 int64_t h3q_quant_per_head_workspace_floats(int64_t batch, int64_t seq, int64_t heads, int64_t head_dim);
 int h3q_quant_per_head_e4m3(const void* x, int64_t batch, int64_t seq, int64_t heads, int64_t head_dim,

@@ -383,8 +383,8 @@ __attribute__((visibility("default"))) int h3q_scaled_mm(int format, const void*
         if (ldt * 2 >= (int64_t(1) << 23) || ldlb * 2 >= (int64_t(1) << 23))
             return fail(H3Q_ERR_UNSUPPORTED, "%s: LoRA row stride above 8 MiB", who);
     }
-    // Tiled activations beyond the weight-streaming GEMM's rows are read by the
-    // four-wave GEMM only (see w4_supported).
+    // Above 128 rows only the streaming and four-wave GEMMs read tiled activations: the
+    // shapes that the latter takes (see w4_supported).
     if (a_tiled && m > h3q::kSkinnyMaxM && (k < 256 || n % 8 || ldo % 8 || !aligned(out, 16) || out_f16))
         return fail(H3Q_ERR_UNSUPPORTED,
                     "%s: tiled activations with m > %lld need k >= 256, n and ldo multiples of 8, a 16-byte "

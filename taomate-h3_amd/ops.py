@@ -287,9 +287,9 @@ def quant_activations_for(x: torch.Tensor, fmt: int, rounding: int, weight: torc
                           lora: bool = False, tiled: bool | None = None):
     """Per-token quantization of the 2-D activations of a linear whose weight
     codes are ``weight`` (bf16 output): tiled when the weight is tiled and the
-    GEMM reads tiled activations at this shape -- the weight-streaming GEMM
-    for at most 128 tokens (no LoRA), the four-wave GEMM above that (K >= 256,
-    N a multiple of 8, with or without the LoRA epilogue) -- else row-major.
+    GEMM reads tiled activations at this shape -- without LoRA for at most 128
+    tokens, with or without it above that (K >= 256, N a multiple of 8) -- else
+    row-major.
     Returns (codes, scales, a_tiled); ``codes`` may be a larger workspace
     buffer of rows >= tiled_rows(m).  ``tiled``: ``is_tiled(weight)`` where the
     caller has it."""

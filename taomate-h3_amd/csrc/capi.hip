@@ -416,6 +416,11 @@ __attribute__((visibility("default"))) int h3q_scaled_mm(int format, const void*
     g.a_tiled = a_tiled;
     g.b_tiled = b_tiled;
     g.out_f16 = out_f16;
+    if (a_tiled && h3q::gemm_plan(g).kernel == h3q::kGemmPerTile)
+        return fail(H3Q_ERR_UNSUPPORTED,
+                    "%s: tiled activations with m <= %lld and row-major weights need n and ldo multiples of 8, a "
+                    "16-byte aligned output and a 4-byte aligned bias",
+                    who, (long long)h3q::kSkinnyMaxM);
     const int kind = format == H3Q_FMT_E4M3FN ? h3q::kOpE4M3 : h3q::kOpInt8;
     return check_launch(h3q::launch_gemm(kind, false, g, (hipStream_t)stream), who);
 }

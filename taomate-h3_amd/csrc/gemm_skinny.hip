@@ -444,6 +444,7 @@ hipError_t launch_skinny_op(const GemmArgs& a, hipStream_t st) {
 
 bool skinny_supported(const GemmArgs& a) {
     const int64_t a_bytes = a.a_tiled ? (a.m + 15) / 16 * (a.k / 128) * 2048 : a.m * a.lda;
+    if (a.a_tiled && !a.b_tiled) return false;  // the row-major weights' kernel reads row-major activations
     return a.m >= 1 && a.m <= kSkinnyMaxM && a.lora_t == nullptr && a_bytes < (int64_t)kOob &&
            a.m * a.ldo * 2 < (int64_t)kOob;
 }

@@ -139,8 +139,9 @@ int stream_tile(const GemmArgs& a) {
         return best.cost < 0.78 * four_wave_cost(a) ? best.tile : 0;
     }
     // M <= 128: against the kernels of gemm_skinny.hip, which take no adapter
-    // (M = 40, 10752 x 5376, rank 64: 61 us by the per-tile kernel).
-    if (a.lora_t || (a.b_tiled ? beats_skinny_tiled(a.m, a.n, a.k) : beats_skinny_rows(a.m, a.n, a.k))) return best.tile;
+    // (M = 40, 10752 x 5376, rank 64: 61 us by the per-tile kernel) and read tiled
+    // activations beside tiled weights only.
+    if (a.lora_t || (a.a_tiled && !a.b_tiled) || (a.b_tiled ? beats_skinny_tiled(a.m, a.n, a.k) : beats_skinny_rows(a.m, a.n, a.k))) return best.tile;
     return 0;
 }
 

@@ -39,6 +39,13 @@ def test_few_rows_row_major_weights(m, n, k, kernel):
     assert gemm_plan(m, n, k)[0] == kernel
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 8, 128), (32, 1024, 3072), (128, 2048, 2048), (16, 5120, 5120)])
+def test_few_rows_of_tiled_activations_on_row_major_weights(m, n, k):
+    """The few-rows kernel of row-major weights reads row-major activations only."""
+    assert gemm_plan(m, n, k, a_tiled=True)[0] == STREAM
+    assert gemm_plan(m, n + 4, k, a_tiled=True)[0] == "per tile"  # h3q_scaled_mm refuses it
+
+
 def test_few_rows_with_an_adapter():
     """The few-rows kernels take no adapter: streaming tiles where their form allows, else per tile."""
     assert gemm_plan(16, 5120, 5120, b_tiled=True, rank=64)[0] == STREAM

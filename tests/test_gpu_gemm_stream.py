@@ -146,3 +146,13 @@ def test_bias_at_an_odd_element(ops, oracle, device, m, n, k):
     exact = sa.cpu().numpy().astype(np.float64)[:, None] * v + packed[1:].double().numpy()
     ref = exact.astype(np.float32).astype(np.float16)  # one rounding each: s_w * acc, the fma
     np.testing.assert_array_equal(out.cpu().numpy().view(np.uint16), ref.view(np.uint16))
+
+
+@pytest.mark.parametrize("m,n,k", [(5, 520, 256), (16, 264, 3072), (33, 1032, 640), (128, 264, 2048)])
+@pytest.mark.parametrize("fmt", ["int8", "e4m3"])
+def test_few_tiled_rows_on_row_major_weights(ops, oracle, device, m, n, k, fmt):
+    """Tiled activations beside row-major weights up to 128 rows; refused where no kernel reads them so."""
+    test_stream_gemm(ops, oracle, device, m, n, k, True, False, fmt)
+    _, _, qa, sa, qw, sw = _operands(ops, device, m, n, k, fmt, True, False)
+    with pytest.raises(RuntimeError, match="row-major weights"):
+        ops.scaled_mm(qa, qw[:n - 4], sa, sw[:n - 4], a_tiled=True, m=m, n=n - 4)
